@@ -576,7 +576,7 @@ __device__ __forceinline__ void fast_tile(const GemmArgs& g, int pid, const int 
   constexpr int WGN = 4 / WGM;
   constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
   static_assert(WGM * WGN == 4 && TM >= 1 && TN >= 1, "wave grid");
-  static_assert(NS == 3 || NS == 4, "three or four LDS stages");
+  static_assert(NS == 3, "three LDS stages");
   constexpr int IA = BM * CPR / 64, IB = BN * CPR / 64;  // wave instructions (KiB) per operand per stage
   static_assert(IA % 4 == 0 && IB % 4 == 0, "each wave issues an equal share of a stage");
   constexpr int JA = IA / 4, JB = IB / 4, G = JA + JB;   // per-wave loads per stage
@@ -588,7 +588,6 @@ __device__ __forceinline__ void fast_tile(const GemmArgs& g, int pid, const int 
   __shared__ __attribute__((aligned(1024))) int8_t L0[ARR];
   __shared__ __attribute__((aligned(1024))) int8_t L1[ARR];
   __shared__ __attribute__((aligned(1024))) int8_t L2[ARR];
-  __shared__ __attribute__((aligned(1024))) int8_t L3[NS == 4 ? ARR : 16];
   __shared__ int8_t lut_s[256];
 
   const int t = threadIdx.x;
@@ -703,12 +702,11 @@ __device__ __forceinline__ void fast_tile(const GemmArgs& g, int pid, const int 
 
   issue(L0, 0);
   issue(L1, BK);
-  if (NS == 4) issue(L2, 2 * BK);
   wait_vm_lgkm0<(NS - 2) * G>();
   stage_barrier();
   load_frags(0, L0, 0);
   int kt = 0;
-  if (NS == 3 && KFULL) {
+  if (KFULL) {
     // KFULL launches have nk % 3 == 0: whole rotations and no tail steps, so the accumulators reach the epilogue from
     // one place (tail steps leave several, and the compiler then copies every accumulator where they join)
     for (; kt < nk; kt += 3) {
@@ -716,7 +714,7 @@ __device__ __forceinline__ void fast_tile(const GemmArgs& g, int pid, const int 
       step(kt + 1, L1, L0, L2);
       step(kt + 2, L2, L1, L0);
     }
-  } else if (NS == 3) {
+  } else {
     for (; kt + 3 <= nk; kt += 3) {
       step(kt, L0, L2, L1);
       step(kt + 1, L1, L0, L2);
@@ -724,16 +722,6 @@ __device__ __forceinline__ void fast_tile(const GemmArgs& g, int pid, const int 
     }
     if (kt < nk) step(kt, L0, L2, L1);
     if (kt + 1 < nk) step(kt + 1, L1, L0, L2);
-  } else {
-    for (; kt + 4 <= nk; kt += 4) {
-      step(kt, L0, L3, L1);
-      step(kt + 1, L1, L0, L2);
-      step(kt + 2, L2, L1, L3);
-      step(kt + 3, L3, L2, L0);
-    }
-    if (kt < nk) step(kt, L0, L3, L1);
-    if (kt + 1 < nk) step(kt + 1, L1, L0, L2);
-    if (kt + 2 < nk) step(kt + 2, L2, L1, L3);
   }
   if constexpr (SPLIT) {
     splitk_finish<BM, BN, WM, WN, TM, TN, OSZ, MUL24>(g, acc, lut_s, tile_m * g.tiles_n + tile_n, m0, n0,
@@ -778,8 +766,7 @@ __device__ __forceinline__ void fast_tile(const GemmArgs& g, int pid, const int 
   auto srow = [&](int r) -> int8_t* {
     if (r < RPA) return L0 + r * SROW;
     if (r < 2 * RPA) return L1 + (r - RPA) * SROW;
-    if (NS == 3 || r < 3 * RPA) return L2 + (r - 2 * RPA) * SROW;
-    return L3 + (r - 3 * RPA) * SROW;
+    return L2 + (r - 2 * RPA) * SROW;
   };
   // the LUT choice is made once, outside the loops: a per-element branch would split the requant into basic blocks
   // that each wait for their LDS reads
@@ -1320,8 +1307,8 @@ static void launch_persist(GemmArgs& g, int osz, int batch, int num_cu, hipStrea
 }
 
 // KF: the shapes the planner takes (256 x 128 and 128 x 128, three stages) have a KFULL form, used when K is a whole
-// number of stage rotations (K % 192 == 0) and not truncated per tile (causal mode 2); the benchmarking-override
-// shapes keep the per-lane K bound
+// number of stage rotations (K % 192 == 0) and not truncated per tile (causal mode 2); 256 x 192 keeps the per-lane K
+// bound
 template <int BM, int BN, int WGM, int NS, bool MUL24, bool KF = false>
 static void launch_fast(GemmArgs& g, int osz, int batch, hipStream_t s) {
   g.tiles_m = (g.M + BM - 1) / BM;
@@ -1785,16 +1772,16 @@ static bool splitk_plan(const GemmArgs& g, int batch, int num_cu, bool force, in
   return force || splits >= 2;
 }
 
-// The fast-path configuration of a product, named by the context's benchmarking override values: 39 and 40 the
-// persistent 256 x 256 (K blocks of 64) and 256 x 128 (K blocks of 128) kernels, 11 - 20 the one-tile-per-workgroup
-// shapes of the switch in launch_fast_choice. An override the product cannot take falls through to the rules.
+// The fast-path configuration of a product, named by the context's benchmarking override values: 39, 40 and 41 the
+// persistent 256 x 256 (K blocks of 64), 256 x 128 and 256 x 256 (K blocks of 128) kernels, 13, 16 and 19 the
+// one-tile-per-workgroup shapes of launch_fast_choice. An override the product cannot take falls through to the rules.
 static int fast_choice(const GemmArgs& g, int batch, int cfg, int num_cu) {
   // the persistent 256 x 256 kernel: one workgroup of 8 waves per CU, four 32 KiB LDS stages, wave tiles 64 x 128
   const bool persist_ok = g.causal == 0 && ((g.K + 63) / 64) % 4 == 0;
   const bool persist128_ok = g.causal == 0 && ((g.K + 127) / 128) % 3 == 0;
   const bool persist128x2_ok = g.causal == 0 && ((g.K + 127) / 128) % 2 == 0;
-  if ((cfg == 39 && persist_ok) || (cfg == 40 && persist128_ok) || ((cfg == 41 || cfg == 42) && persist128x2_ok) ||
-      (cfg >= 11 && cfg <= 20))
+  if ((cfg == 39 && persist_ok) || (cfg == 40 && persist128_ok) || (cfg == 41 && persist128x2_ok) || cfg == 13 ||
+      cfg == 16 || cfg == 19)
     return cfg;
   // measured on MI355X (block GEMM shapes, K 768 and 3072): wide products with at least six 256 x 256 tiles per CU
   // take the persistent kernel (it halves the L2 traffic per MFMA of the 256 x 128 tile); 256 x 128 tiles with three
@@ -1829,16 +1816,8 @@ static void launch_fast_choice(GemmArgs& g, int osz, int batch, hipStream_t s, i
     case 39: return launch_persist<256, 256, 64, 4, MUL24, 8, 2>(g, osz, batch, num_cu, s);
     case 40: return launch_persist<256, 128, 128, 3, MUL24, 8, 2>(g, osz, batch, num_cu, s);
     case 41: return launch_persist<256, 256, 128, 2, MUL24, 8, 2>(g, osz, batch, num_cu, s);
-    case 42: return launch_persist<256, 128, 128, 2, MUL24, 8, 2>(g, osz, batch, num_cu, s);
-    case 11: return launch_fast<256, 256, 2, 3, MUL24>(g, osz, batch, s);
-    case 12: return launch_fast<256, 256, 2, 4, MUL24>(g, osz, batch, s);
-    case 14: return launch_fast<128, 128, 2, 4, MUL24>(g, osz, batch, s);
-    case 15: return launch_fast<256, 128, 2, 4, MUL24>(g, osz, batch, s);
     case 16: return launch_fast<256, 128, 2, 3, MUL24, true>(g, osz, batch, s);
-    case 17: return launch_fast<128, 256, 2, 3, MUL24>(g, osz, batch, s);
-    case 18: return launch_fast<128, 192, 2, 3, MUL24>(g, osz, batch, s);
     case 19: return launch_fast<256, 192, 2, 3, MUL24>(g, osz, batch, s);
-    case 20: return launch_fast<256, 192, 2, 4, MUL24>(g, osz, batch, s);
     default: return launch_fast<128, 128, 2, 3, MUL24, true>(g, osz, batch, s);
   }
 }
@@ -1863,18 +1842,8 @@ static void launch_cfg(GemmArgs& g, int osz, bool vec, int batch, hipStream_t s)
 
 // Tile shape by problem: 128 x 128 for checked runs (its epilogue keeps the 64-bit checks in registers) and small
 // problems, 256 x 64 with the four waves stacked along M when N <= 64 (attention's P.V), 256 x 256 otherwise.
-// cfg (the context's ANVIL_GEMM_CFG, a benchmarking override) pins one shape for every unchecked GEMM.
-static void launch_gemm(GemmArgs& g, bool checked, int osz, bool vec, int batch, hipStream_t s, int cfg) {
+static void launch_gemm(GemmArgs& g, bool checked, int osz, bool vec, int batch, hipStream_t s) {
   if (checked) return launch_cfg<128, 128, 64, 2, 1, true>(g, osz, vec, batch, s);
-  switch (cfg) {
-    case 1: return launch_cfg<256, 256, 64, 2, 1, false>(g, osz, vec, batch, s);
-    case 2: return launch_cfg<256, 256, 64, 2, 2, false>(g, osz, vec, batch, s);
-    case 3: return launch_cfg<256, 128, 64, 2, 2, false>(g, osz, vec, batch, s);
-    case 4: return launch_cfg<128, 128, 64, 2, 2, false>(g, osz, vec, batch, s);
-    case 5: return launch_cfg<256, 256, 128, 2, 1, false>(g, osz, vec, batch, s);
-    case 6: return launch_cfg<128, 256, 64, 2, 2, false>(g, osz, vec, batch, s);
-    default: break;
-  }
   if (g.N <= 64)
     launch_cfg<256, 64, 64, 4, 2, false>(g, osz, vec, batch, s);
   else if (g.M <= 128 || g.N <= 128)
@@ -2032,8 +2001,7 @@ static int gemm_prepare(anvil_ctx* ctx, const int8_t* A, const int8_t* Bt, void*
                 (batch1 == 1 || ok16(g.sc1 * osz));
   if ((long long)((M + 127) / 128) * ((N + 63) / 64) > (1ll << 31) - 1)
     return set_error(ANVIL_E_VALUE, "anvil_gemm_i8: too many tiles");
-  const bool force_generic = !add && ctx->gemm_cfg >= 1 && ctx->gemm_cfg <= 6;   // benchmarking override
-  const bool fast = !checked && vec && !force_generic && 256ll * g.lda < (1ll << 31) && 256ll * g.ldb < (1ll << 31);
+  const bool fast = !checked && vec && 256ll * g.lda < (1ll << 31) && 256ll * g.ldb < (1ll << 31);
   if (add) {
     if (!fast)
       return set_error(ANVIL_E_VALUE, "anvil_gemm_i8_add: operands must be 16-byte aligned with K a multiple of 16");
@@ -2059,7 +2027,7 @@ static int gemm_prepare(anvil_ctx* ctx, const int8_t* A, const int8_t* Bt, void*
   p.force_split = (flags & ANVIL_GEMM_SPLITK) != 0;
   if ((flags & (ANVIL_GEMM_A_KBLOCK | ANVIL_GEMM_B_KBLOCK | ANVIL_GEMM_C_KBLOCK)) && !fast)
     return set_error(ANVIL_E_VALUE, "anvil_gemm_i8: K-blocked operands need 16-byte aligned operands with K a multiple "
-                                    "of 16 (and no benchmarking override)");
+                                    "of 16");
   if (p.force_split && !fast)
     return set_error(ANVIL_E_VALUE, "anvil_gemm_i8: SPLITK needs 16-byte aligned operands with K a multiple of 16");
   return ANVIL_OK;
@@ -2081,7 +2049,7 @@ static int ensure_workspace(anvil_ctx* ctx, long long sums) {
 // first use), or with `noalloc` in the static scratch, within whose size it must then fit.
 static int gemm_launch(anvil_ctx* ctx, Prepared& p, bool noalloc = false) {
   if (!p.fast) {
-    launch_gemm(p.g, p.checked, p.osz, p.vec, p.batch, ctx->stream, ctx->gemm_cfg);
+    launch_gemm(p.g, p.checked, p.osz, p.vec, p.batch, ctx->stream);
     return ANVIL_OK;
   }
   int splits = 0, kchunk = 0;
