@@ -111,6 +111,8 @@ class _Plan:
         self.stage: dict = {}          # device staging buffers of float inputs and token ids
         self.host_stage: dict = {}     # page-locked host buffers the read-back downloads into, by device buffer
         self.graph = None              # the steps captured as one HIP graph (run(..., graph=True))
+        self.launched = False          # an eager launch has run
+        self.sequence = None           # the kernels of the plan's second eager launch, for the next ones
         self.eager_ms: list = []       # device ms of the plan's first eager runs (run's default launch choice)
         self.graph_ms = None           # device ms of its first replay of the captured graph
         self.replay = None             # run's choice once measured: True = replay the graph, False = launch eagerly
@@ -1011,9 +1013,11 @@ class CompiledModel:
         return b
 
     def launch(self, plan, profile=False, graph=False):
-        """Enqueue every kernel of the plan on the device stream (asynchronous unless profile). graph=True replays
-        the steps as one HIP graph, captured on the plan's first such launch right after an ordinary launch of the
-        same steps (which allocates every workspace they need, so the capture records kernels only)."""
+        """Enqueue every kernel of the plan on the device stream (asynchronous unless profile). The plan's
+        first two launches call its steps one by one, the second recording the kernels they launch (Device.sequence);
+        the next ones issue those kernels in one native call. graph=True replays the steps as captured on the plan's first such launch, right
+        after an ordinary launch of the same steps (which allocates every workspace they need, so the capture records
+        kernels only)."""
         times = {}
         if not profile and graph:
             if plan.graph is None:
@@ -1022,7 +1026,13 @@ class CompiledModel:
             plan.graph.launch()
             return times
         if not profile:
-            _launch_steps(plan)
+            if plan.sequence is not None:
+                plan.sequence.launch()
+            elif plan.launched and isinstance(self.dev, rt.Device):   # a stand-in device records no kernels
+                plan.sequence = self.dev.sequence(_launch_steps, plan)
+            else:
+                _launch_steps(plan)
+                plan.launched = True
             return times
         # each step's kernels carry their own pair of events (anvil_time_kernels): device time of the kernels alone
         for label, fn, args in plan.steps:

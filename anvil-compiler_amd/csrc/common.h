@@ -68,16 +68,23 @@ struct KernelTimer {
 };
 extern __thread KernelTimer g_timer;   // zero-initialised per thread (a trivial type: no TLS init function)
 
-#define ANVIL_LAUNCH(kernel, grid, block, lds, strm_, ...)                                                  \
-  do {                                                                                                      \
-    if (::anvil::g_timer.stop && ::anvil::g_timer.stream == (strm_)) {                                      \
-      hipEvent_t start_ = ::anvil::g_timer.start;                                                           \
-      ::anvil::g_timer.start = nullptr;                                                                     \
-      hipExtLaunchKernelGGL(kernel, grid, block, lds, strm_, start_, ::anvil::g_timer.stop, 0, __VA_ARGS__); \
-    } else {                                                                                                \
-      hipLaunchKernelGGL(kernel, grid, block, lds, strm_, __VA_ARGS__);                                     \
-    }                                                                                                       \
-  } while (0)
+// Every kernel goes out through launch_kernel: with the timer's events while it is armed for the stream, and noted in
+// the launch list that this thread is recording on the stream, if any (anvil_graph_begin, anvil_record_begin).
+int launch_kernel(const void* fn, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
+                  const unsigned short* sizes, int n);
+
+template <typename T>
+struct as_is { using type = T; };
+
+template <typename... P>
+void launch(void (*kernel)(P...), dim3 grid, dim3 block, unsigned lds, hipStream_t s, typename as_is<P>::type... args) {
+  static constexpr unsigned short sizes[] = {(unsigned short)sizeof(P)...};
+  void* ptrs[] = {(void*)&args...};
+  launch_kernel(reinterpret_cast<const void*>(kernel), grid, block, lds, s, ptrs, sizes, (int)sizeof...(P));
+}
+
+#define ANVIL_LAUNCH(kernel, grid, block, lds, strm_, ...) \
+  ::anvil::launch(kernel, grid, block, (unsigned)(lds), strm_, __VA_ARGS__)
 
 #define ANVIL_LAUNCHED()                                                      \
   do {                                                                        \

@@ -2,6 +2,8 @@
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
+#include <utility>
+#include <vector>
 
 #include "common.h"
 
@@ -9,6 +11,66 @@ namespace anvil {
 
 static thread_local std::string g_last_error;
 __thread KernelTimer g_timer;
+
+// A recorded launch: the kernel and a copy of its arguments (ptrs into bytes).
+struct LaunchRecord {
+  const void* sym;
+  hipFunction_t fn;
+  dim3 grid, block;
+  unsigned lds;
+  std::vector<char> bytes;
+  std::vector<void*> ptrs;
+  std::vector<unsigned short> sizes;
+};
+
+// What anvil_graph_end and anvil_record_end return: the recorded launches, or (exec set) a captured HIP graph whose
+// nodes are not all launches that the capturing thread made through launch_kernel.
+struct LaunchList {
+  std::vector<LaunchRecord> launches;
+  hipGraphExec_t exec = nullptr;
+};
+
+// the lists this thread is recording, innermost last, each with the stream it records
+struct Recording {
+  hipStream_t stream;
+  LaunchList* list;
+};
+static thread_local std::vector<Recording> g_recordings;
+
+static hipError_t note_launch(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
+                              const unsigned short* sizes, int n) {
+  for (Recording& rec : g_recordings) {
+    if (rec.stream != s) continue;
+    LaunchRecord r{sym, nullptr, grid, block, lds, {}, {}, {sizes, sizes + n}};
+    if (hipError_t e = hipGetFuncBySymbol(&r.fn, sym); e != hipSuccess) return e;
+    size_t total = 0;
+    for (int i = 0; i < n; ++i) total = (total + 15) / 16 * 16 + sizes[i];
+    r.bytes.resize(total + 1);
+    size_t at = 0;
+    for (int i = 0; i < n; ++i) {
+      at = (at + 15) / 16 * 16;
+      std::memcpy(r.bytes.data() + at, args[i], sizes[i]);
+      r.ptrs.push_back(r.bytes.data() + at);
+      at += sizes[i];
+    }
+    rec.list->launches.push_back(std::move(r));   // moving the vectors keeps their storage, and so the pointers
+  }
+  return hipSuccess;
+}
+
+int launch_kernel(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
+                  const unsigned short* sizes, int n) {
+  hipError_t e;
+  if (g_timer.stop && g_timer.stream == s) {
+    hipEvent_t start = g_timer.start;
+    g_timer.start = nullptr;
+    e = hipExtLaunchKernel(sym, grid, block, args, lds, s, start, g_timer.stop, 0);
+  } else {
+    e = hipLaunchKernel(sym, grid, block, args, lds, s);
+  }
+  if (e == hipSuccess && !g_recordings.empty()) e = note_launch(sym, grid, block, lds, s, args, sizes, n);
+  return e == hipSuccess ? ANVIL_OK : hip_fail(e, "kernel launch");
+}
 
 int set_error(int code, const char* fmt, ...) {
   char buf[1024];
@@ -181,39 +243,107 @@ int anvil_zero(anvil_ctx* ctx, void* dst, size_t bytes) {
   return zero_fill(ctx->stream, dst, bytes);
 }
 
+// Recordings start and end on one thread; they nest.
+static void record_start(anvil_ctx* ctx) { g_recordings.push_back({ctx->stream, new LaunchList()}); }
+
+static LaunchList* record_stop(anvil_ctx* ctx) {
+  if (g_recordings.empty() || g_recordings.back().stream != ctx->stream) return nullptr;
+  LaunchList* l = g_recordings.back().list;
+  g_recordings.pop_back();
+  return l;
+}
+
 int anvil_graph_begin(anvil_ctx* ctx) {
   if (int r = check_ctx(ctx)) return r;
   ANVIL_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
+  record_start(ctx);
   return ANVIL_OK;
 }
 
 int anvil_graph_end(anvil_ctx* ctx, void** graph) {
   if (int r = check_ctx(ctx)) return r;
-  if (!graph) return set_error(ANVIL_E_VALUE, "anvil_graph_end: null output pointer");
+  LaunchList* l = record_stop(ctx);
+  if (!graph) {
+    delete l;
+    return set_error(ANVIL_E_VALUE, "anvil_graph_end: null output pointer");
+  }
   *graph = nullptr;
   hipGraph_t g = nullptr;
-  ANVIL_HIP(hipStreamEndCapture(ctx->stream, &g));       // ends the capture whatever happened inside it
-  hipGraphExec_t exec = nullptr;
-  const hipError_t e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+  hipError_t e = hipStreamEndCapture(ctx->stream, &g);   // ends the capture whatever happened inside it
+  if (e != hipSuccess) {
+    delete l;
+    return hip_fail(e, "hipStreamEndCapture(ctx->stream, &g)");
+  }
+  // The captured nodes are this thread's recorded launches, one after another on one stream: they are replayed as
+  // launches from the list. hipGraphLaunch of the same kernels costs more on both sides: 28 us of host time for one
+  // node to 43 us for twelve, and about 0.7 us more a node on the device (measured: a 768-wide block on one sequence,
+  // 7 nodes, 61.4 us a forward through hipGraphLaunch, 55 us as launches; the 128-wide two-layer model, 12 nodes,
+  // 96.5 against 89.7 us). A graph that holds anything else keeps its executable form.
+  size_t nodes = 0;
+  e = hipGraphGetNodes(g, nullptr, &nodes);
+  if (!l) l = new LaunchList();
+  if (e != hipSuccess || nodes != l->launches.size()) {
+    l->launches.clear();
+    e = hipGraphInstantiate(&l->exec, g, nullptr, nullptr, 0);
+  }
   hipGraphDestroy(g);
-  if (e != hipSuccess) return ::anvil::hip_fail(e, "hipGraphInstantiate");
-  *graph = exec;
+  if (e != hipSuccess) {
+    delete l;
+    return hip_fail(e, "hipGraphInstantiate");
+  }
+  *graph = l;
   return ANVIL_OK;
+}
+
+int anvil_record_begin(anvil_ctx* ctx) {
+  if (int r = check_ctx(ctx)) return r;
+  record_start(ctx);
+  return ANVIL_OK;
+}
+
+int anvil_record_end(anvil_ctx* ctx, void** list) {
+  if (int r = check_ctx(ctx)) return r;
+  LaunchList* l = record_stop(ctx);
+  if (!list) {
+    delete l;
+    return set_error(ANVIL_E_VALUE, "anvil_record_end: null output pointer");
+  }
+  *list = l;
+  return l ? ANVIL_OK : set_error(ANVIL_E_VALUE, "anvil_record_end: nothing is being recorded on this thread");
 }
 
 int anvil_graph_launch(anvil_ctx* ctx, void* graph) {
   if (int r = check_ctx(ctx)) return r;
   if (!graph) return set_error(ANVIL_E_VALUE, "anvil_graph_launch: null graph");
-  ANVIL_HIP(hipGraphLaunch((hipGraphExec_t)graph, ctx->stream));
+  LaunchList* l = (LaunchList*)graph;
+  if (l->exec) {
+    ANVIL_HIP(hipGraphLaunch(l->exec, ctx->stream));
+    return ANVIL_OK;
+  }
+  const bool plain = g_recordings.empty() && !(g_timer.stop && g_timer.stream == ctx->stream);
+  for (LaunchRecord& r : l->launches) {
+    if (plain) {
+      ANVIL_HIP(hipModuleLaunchKernel(r.fn, r.grid.x, r.grid.y, r.grid.z, r.block.x, r.block.y, r.block.z, r.lds,
+                                      ctx->stream, r.ptrs.data(), nullptr));
+    } else if (int e = launch_kernel(r.sym, r.grid, r.block, r.lds, ctx->stream, r.ptrs.data(), r.sizes.data(),
+                                     (int)r.sizes.size())) {
+      return e;
+    }
+  }
   return ANVIL_OK;
 }
 
 int anvil_graph_destroy(anvil_ctx* ctx, void* graph) {
   if (int r = check_ctx(ctx)) return r;
   if (!graph) return ANVIL_OK;
-  ANVIL_HIP(hipStreamSynchronize(ctx->stream));
-  ANVIL_HIP(hipGraphExecDestroy((hipGraphExec_t)graph));
-  return ANVIL_OK;
+  LaunchList* l = (LaunchList*)graph;
+  hipError_t e = hipSuccess;
+  if (l->exec) {
+    e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = hipGraphExecDestroy(l->exec);
+  }
+  delete l;
+  return e == hipSuccess ? ANVIL_OK : hip_fail(e, "hipGraphExecDestroy");
 }
 
 // The context's events only time work (anvil_event_elapsed, anvil_time_kernels); nothing reads device memory through
