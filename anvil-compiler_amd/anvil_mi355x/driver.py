@@ -128,6 +128,12 @@ class _Plan:
         b = self.buf(math.prod(dims) * rt.ITEMSIZE[dtype], name)
         return View(b, dtype, dims, contig_strides(dims))
 
+    def padded(self, dims, dtype, row, name=""):
+        """Storage whose last dim takes `row` >= dims[-1] elements."""
+        dims = tuple(int(d) for d in dims)
+        b = self.buf(math.prod(dims[:-1]) * row * rt.ITEMSIZE[dtype], name)
+        return View(b, dtype, dims, contig_strides((*dims[:-1], row)))
+
     def kblocked(self, dims, dtype, name=""):
         """Storage for a value read only as a GEMM operand: the last dim in 64-element blocks, each block holding
         all rows consecutively (block stride rows * 64)."""
@@ -204,8 +210,8 @@ class CompiledModel:
 
     def _chain_of(self, o_op):
         """(scores matmul, softmax) when o_op is the P.V product of a chain the fused attention evaluates (the
-        structure only: proven, int8 throughout, scores and p read by nothing else, square scores with T a multiple
-        of 32 up to 1024 and a head dim of 16, 32, 64 or 128, or T = 16 and a head dim of 16 or 32), else None."""
+        structure only: proven, int8 throughout, scores and p read by nothing else, square scores with T up to 1024
+        and a head dim of 16, 32, 64 or 128), else None."""
         if not self.proven or not isinstance(o_op, g.QMatmulOp) or o_op.lut is not None:
             return None
         if g.qt(o_op.result).dtype != "i8":
@@ -221,14 +227,14 @@ class CompiledModel:
             return None
         sd, od = g.qt(s_op.result).dims, g.qt(o_op.result).dims
         T, D = sd[-1], g.qt(s_op.a).dims[-1]
-        if (sd[-2] != T or (T % 32 and T != 16) or T > 1024 or D not in (16, 32, 64, 128) or (T == 16 and D > 32)
-                or od[-1] != D or od[-2] != T):
+        if sd[-2] != T or T > 1024 or D not in (16, 32, 64, 128) or od[-1] != D or od[-2] != T:
             return None
         return s_op, sm
 
     def _t16_chain(self, o_op) -> bool:
+        """A chain of the T = 16 kernel (heads of 16 or 32), which takes V's rows or V^T's."""
         chain = self._chain_of(o_op)
-        return chain is not None and g.qt(chain[0].result).dims[-1] == 16
+        return chain is not None and g.qt(chain[0].result).dims[-1] == 16 and g.qt(o_op.result).dims[-1] <= 32
 
     def _const_array(self, v):
         """The int64 values of a graph const, None for a computed value."""
@@ -426,8 +432,7 @@ class CompiledModel:
     def _attention_chains(self, keep) -> dict:
         """{P.V matmul: (scores matmul, softmax)} for every chain qmatmul -> softmax_lut -> qmatmul whose scores and
         probabilities are read by nothing else, in a proven graph with int8 values throughout, a square (T x T)
-        score matrix with T a multiple of 32 up to 1024 and one head dim of 16, 32, 64 or 128, or T = 16 and a head
-        dim of 16 or 32: the chains
+        score matrix with T up to 1024 and one head dim of 16, 32, 64 or 128: the chains
         anvil_attention_i8 evaluates without materialising scores or p, or, when the run returns them (keep="all",
         or graph outputs), anvil_attention_i8_keep, which also stores them (_kept_chain)."""
         if not self.proven:
@@ -452,7 +457,8 @@ class CompiledModel:
         kb = views[s_op.b].permute(_swap_last2(n))           # key rows (..., T, d)
         vb = views[o_op.b].permute(_swap_last2(n))           # V^T rows (..., d, T)
         T0 = g.qt(s_op.result).dims[-1]
-        vrows = T0 == 16 and vb.strides[-1] != 1 and views[o_op.b].strides[-1] == 1
+        t16 = self._t16_chain(o_op)
+        vrows = t16 and vb.strides[-1] != 1 and views[o_op.b].strides[-1] == 1
         if vrows:                                           # the T = 16 kernel takes V's own rows (..., T, d)
             vb = views[o_op.b]
         om = self._merged_heads(o_op)
@@ -467,8 +473,12 @@ class CompiledModel:
             out = self._alloc_result(P, o_op, (nb, *g.qt(o_op.result).dims), label)
         vs = [qa, kb, vb, out]
         if kept:
-            sv = self._alloc_result(P, s_op, (nb, *g.qt(s_op.result).dims), label + ".scores")
-            pv = P.dense((nb, *g.qt(sm.result).dims), "i8", label + ".p")
+            row = T0 if t16 else -(-T0 // 32) * 32           # whole 32-key tiles are stored
+            if row == T0:
+                sv = self._alloc_result(P, s_op, (nb, *g.qt(s_op.result).dims), label + ".scores")
+            else:
+                sv = P.padded((nb, *g.qt(s_op.result).dims), "i8", row, label + ".scores")
+            pv = P.padded((nb, *g.qt(sm.result).dims), "i8", row, label + ".p")
             vs += [sv, pv]
         lead = out.dims[:-2]
         idx = [i for i, d in enumerate(lead) if d != 1]
@@ -486,11 +496,11 @@ class CompiledModel:
             vrow_len, vrows_n = (D, T) if vrows else (T, D)   # V rows (T of D keys' values) or V^T rows
             fits = (all(st % 16 == 0 for st in strides[:9]) and all(st % 4 == 0 for st in strides[9:12])
                     and all(o % 16 == 0 for o in offs[:3]) and offs[3] % 4 == 0
-                    and strides[5] >= D and strides[8] >= vrow_len and T * strides[5] < 1 << 31
+                    and strides[5] >= D and strides[8] >= vrow_len and -(-T // 32) * 32 * strides[5] < 1 << 31
                     and vrows_n * strides[8] < 1 << 31 and strides[11] >= D and 32 * strides[11] < 1 << 31)
             if kept:                     # S and P: 16-byte stores into 32-row tiles through 32-bit offsets
                 fits = (fits and all(st % 16 == 0 for st in strides[12:]) and all(o % 16 == 0 for o in offs[4:])
-                        and all(T <= st and 32 * st < 1 << 31 for st in (strides[14], strides[17])))
+                        and all(row <= st and 32 * st < 1 << 31 for st in (strides[14], strides[17])))
         if not fits:
             sv = self._plan_matmul(P, s_op, views, (nb, *g.qt(s_op.result).dims), label + ".scores", dense, step,
                                    keep)
@@ -502,6 +512,8 @@ class CompiledModel:
         b0, b1 = [1 if i is None else lead[i] for i in idx]
         T, D = qa.dims[-2], qa.dims[-1]
         flags = rt.OP_UNCHECKED | (rt.ATTN_V_ROWS if vrows else 0)
+        if T % 32 and not t16:
+            flags |= rt.ATTN_RAGGED
         if self.acc_bounds.get(s_op.result, 1 << 31) < (1 << 23) and abs(int(s_op.M)) < (1 << 23):
             flags |= rt.ATTN_S24
         if kept:
@@ -523,7 +535,10 @@ class CompiledModel:
             return P.dense(out_dims, t.dtype, label)
         k = 0 if op.result in self.is_const else 1
         pfull = list(range(k)) + [p + k for p in perm]
-        st = P.dense([out_dims[i] for i in pfull], t.dtype, label)
+        dims = [out_dims[i] for i in pfull]
+        # a transposed int8 result (V^T) is read through 16-byte loads of its rows: they start at multiples of 16
+        swapped = list(perm) == _swap_last2(len(perm)) and t.dtype == "i8"
+        st = P.padded(dims, t.dtype, -(-dims[-1] // 16) * 16 if swapped else dims[-1], label)
         return st.permute([pfull.index(i) for i in range(len(pfull))])
 
     def _bt_const(self, op):

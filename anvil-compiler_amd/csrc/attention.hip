@@ -9,6 +9,11 @@
 // held in registers. Nothing is approximated: the LUT softmax is not invariant under rescaling, which rules out an
 // online (single-pass) softmax.
 //
+// T need not be a multiple of 32 (ANVIL_ATTN_RAGGED): the last query tile stores only its rows below T, and the last key
+// tile masks its keys past T as the causal diagonal masks keys past the row. (T = 250, 16 sequences of six heads of 64:
+// scores, softmax and P.V as three launches took 75 us, P.V's K of 250 on byte loads; this kernel takes 11 us, and the
+// block 127 -> 53 us.)
+//
 // Workgroup: 4 waves on 32 query rows q0 .. q0 + 31; wave w takes the 32-key tiles w, w + 4, w + 8, ... up to the
 // causal diagonal, so the waves share the row's keys evenly and each holds at most T / 128 tiles of scores.
 //   1. S = Q K^T per tile on v_mfma_i32_32x32x32_i8, requantised to int8 and kept packed in registers: lane l holds
@@ -54,18 +59,19 @@ struct AttnArgs {
   int mo, so, rndo;    // output requant
   int mo24;            // |mo| < 2^23: the output requant multiply fits 24 bits
   int clo_o, chi_o;    // the output requant's clamp in the pre-shift domain, as clo / chi
-  int ldo32, obytes;   // O's row stride, and the bytes of one 32-row tile (31 ldo + D), both below 2^31
+  int masked;          // the last key tile has keys to mask: causal, or T no multiple of 32
+  int ldo32;           // O's row stride (32 of them below 2^31)
   unsigned long long mone;   // n / one as (n mone) >> (32 + kone)
   int kone;
-  int nqt;             // query tiles of 32 rows per head
+  int nqt;             // query tiles of 32 rows per head (the last one short when T is no multiple of 32)
   unsigned long long mq, mb;   // n / nqt and n / batch1 as (n m) >> (32 + k): m = ceil(2^(32+k) / d), 2^k >= d
   int kq, kb;
   // the kept form (anvil_attention_i8_keep): scores and probabilities also stored, (batch, head, T, T) int8 with
-  // strides (sc0, sc1, ldsc) and (pr0, pr1, ldpr); one 32-row tile spans 31 ld + T bytes of each (scbytes, prbytes)
+  // strides (sc0, sc1, ldsc) and (pr0, pr1, ldpr), the row strides at least 32 nqt
   int8_t* Sc;
   int8_t* Pr;
   long long sc0, sc1, ldsc, pr0, pr1, ldpr;
-  int ldsc32, ldpr32, scbytes, prbytes;
+  int ldsc32, ldpr32;
   int vrows;           // T = 16 only: V given as its (T, D) rows (strides sv0, sv1, ldv) instead of V^T
 };
 
@@ -138,10 +144,13 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
   const int qt = a.nqt - 1 - (pid - bh * a.nqt);
   const int q0 = qt * 32;
   const int b0 = (int)udiv_magic((unsigned)bh, a.mb, a.kb), b1 = bh - b0 * a.batch1;
-  const int qrow = q0 + l32;
   const int ntiles = a.causal ? qt + 1 : a.nqt;
+  // T no multiple of 32: the last query tile has rows past T (computed on the last row's query, never stored), and the
+  // last key tile keys past T (zeros beyond K's descriptor), which every row masks; klast is the row's last kept key
+  const int qrows = min(32, a.T - q0);
+  const int klast = a.causal ? q0 + l32 : a.T - 1;
 
-  const int8_t* Qr = a.Q + b0 * a.sq0 + b1 * a.sq1 + (long long)qrow * a.ldq;
+  const int8_t* Qr = a.Q + b0 * a.sq0 + b1 * a.sq1 + (long long)(q0 + min(l32, qrows - 1)) * a.ldq;
   // key rows enter the score MFMA in bperm order: score accumulator r of lane l is then key 16 (l / 32) + r of the
   // tile, so a lane's 16 probabilities are 16 consecutive keys and its V^T fragment is one contiguous 16-byte load
   const int8_t* Vb = a.V + b0 * a.sv0 + b1 * a.sv1;
@@ -154,9 +163,11 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
   // are keys 16 (l / 32) .. + 15 of row q0 + l % 32 (the key rows entered the score MFMA in bperm order), one
   // 16-byte store at column 32 nt + 16 (l / 32).
   const __amdgpu_buffer_rsrc_t srs =            // (unused, and dropped, in the plain form)
-      uniform_rsrc(KEEP ? a.Sc + b0 * a.sc0 + b1 * a.sc1 + (long long)q0 * a.ldsc : nullptr, KEEP ? a.scbytes : 0);
+      uniform_rsrc(KEEP ? a.Sc + b0 * a.sc0 + b1 * a.sc1 + (long long)q0 * a.ldsc : nullptr,
+                   KEEP ? (qrows - 1) * a.ldsc32 + 32 * a.nqt : 0);
   const __amdgpu_buffer_rsrc_t prs =
-      uniform_rsrc(KEEP ? a.Pr + b0 * a.pr0 + b1 * a.pr1 + (long long)q0 * a.ldpr : nullptr, KEEP ? a.prbytes : 0);
+      uniform_rsrc(KEEP ? a.Pr + b0 * a.pr0 + b1 * a.pr1 + (long long)q0 * a.ldpr : nullptr,
+                   KEEP ? (qrows - 1) * a.ldpr32 + 32 * a.nqt : 0);
   const unsigned sofs = KEEP ? (unsigned)(l32 * a.ldsc32 + 16 * half) : 0u;
   const unsigned pofs = KEEP ? (unsigned)(l32 * a.ldpr32 + 16 * half) : 0u;
 
@@ -238,16 +249,16 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
       const int y = S24 ? __mul24(acc[r], a.ms) + a.rnds : acc[r] * a.ms + a.rnds;
       x[r] = med3i(y, a.clo, a.chi);
     }
-    // the diagonal tile: a key past the row takes the lowest score (clo >> ss), which leaves the row max as it is;
-    // the sums subtract its LUT term and the probabilities mask it
-    if (a.causal && nt == ntiles - 1) {
+    // the last tile (the diagonal one, or one with keys past T): a key past the row's last takes the lowest score
+    // (clo >> ss), which leaves the row max as it is; the sums subtract its LUT term and the probabilities mask it
+    if (a.masked && nt == ntiles - 1) {
       if constexpr (KEEP) {                           // the kept scores are the unmasked ones
         v4i sv;
 #pragma unroll
         for (int g = 0; g < 4; ++g) sv[g] = (int)sra_pack4(x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3], a.ss);
         store16(sv, srs, sofs + 32 * nt);
       }
-      const int lim = qrow - nt * 32 - 16 * half;     // key r of this lane is kept iff r <= lim
+      const int lim = klast - nt * 32 - 16 * half;    // key r of this lane is kept iff r <= lim
 #pragma unroll
       for (int r = 0; r < 16; ++r) x[r] = r <= lim ? x[r] : a.clo;
     }
@@ -259,7 +270,7 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
 #pragma unroll
     for (int g = 0; g < 4; ++g) sc[i][g] = sra_pack4(x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3], a.ss);
     if constexpr (KEEP) {
-      if (!(a.causal && nt == ntiles - 1))
+      if (!(a.masked && nt == ntiles - 1))
         store16(v4i{(int)sc[i][0], (int)sc[i][1], (int)sc[i][2], (int)sc[i][3]}, srs, sofs + 32 * nt);
     }
 
@@ -271,7 +282,9 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
   int mx = max(mxc >> a.ss, -128);
 
   // the first V^T tile loads while the row maxima are reduced and the sums run
-  const __amdgpu_buffer_rsrc_t vrs = uniform_rsrc(Vb, (int)((long long)D * a.ldv));
+  // up to the last row's T keys rounded up to whole 16-byte chunks (at most its ldv bytes): a chunk past T reads the
+  // row's padding or the next row, or zeros beyond the last row's, and meets p = 0
+  const __amdgpu_buffer_rsrc_t vrs = uniform_rsrc(Vb, (int)((D - 1) * a.ldv) + ((a.T + 15) & ~15));
   auto vload = [&](int nt, v4i* vf) {                    // as for K: offsets below D ldv < 2^31, tile part 2^31 past
     const unsigned tile = nt < ntiles ? (unsigned)(nt * 32) : 0x80000000u;
 #pragma unroll
@@ -312,8 +325,8 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
       });
     }
   });
-  if (a.causal && ((ntiles - 1 - w) & 3) == 0 && w < ntiles) {   // this wave holds the diagonal tile: its masked
-    const int lim = l32 - 16 * half;                              // keys (those past r = lim) added lut terms of
+  if (a.masked && ((ntiles - 1 - w) & 3) == 0 && w < ntiles) {   // this wave holds the last tile: its masked keys
+    const int lim = klast - 32 * (ntiles - 1) - 16 * half;        // (those past r = lim) added lut terms of
     S -= (15 - max(-1, min(lim, 15))) * lut_s[(a.clo >> a.ss) + 255 - mx];   // the lowest score
   }
   S += __shfl_xor(S, 32, 64);
@@ -408,9 +421,9 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
       pf[g] = (int)pack4(p[0], p[1], p[2], p[3]);
       if (g == 1) __builtin_amdgcn_sched_barrier(0);  // two halves of eight lookups: 8 registers fewer at the peak
     }
-    if (a.causal && nt == ntiles - 1) {
-      asm volatile("");                                  // keeps the masking on the diagonal tile's own path
-      const int lim = qrow - nt * 32 - 16 * half;        // bytes r <= lim kept: n of dword g's four
+    if (a.masked && nt == ntiles - 1) {
+      asm volatile("");                                  // keeps the masking on the last tile's own path
+      const int lim = klast - nt * 32 - 16 * half;       // bytes r <= lim kept: n of dword g's four
 #pragma unroll
       for (int g = 0; g < 4; ++g) pf[g] &= (int)(0xFFFFFFFFull >> (32 - 8 * min(max(lim + 1 - 4 * g, 0), 4)));
     }
@@ -461,7 +474,8 @@ __global__ __launch_bounds__(A_THREADS, (D <= 64 ? (KEEP ? 5 : 6) : 1)) void att
   // output byte is one shift written into its byte lane; the tile's 32 rows are stored through a buffer descriptor
   // with 32-bit offsets.
   constexpr int C4 = D / 4;                              // 4-column groups per row
-  const __amdgpu_buffer_rsrc_t ors = uniform_rsrc(a.O + b0 * a.so0 + b1 * a.so1 + (long long)q0 * a.ldo, a.obytes);
+  const __amdgpu_buffer_rsrc_t ors = uniform_rsrc(a.O + b0 * a.so0 + b1 * a.so1 + (long long)q0 * a.ldo,
+                                                  (qrows - 1) * a.ldo32 + D);
   auto store = [&](auto m24) {
     for (int idx = t; idx < 32 * C4; idx += A_THREADS) {
       const int row = idx / C4, c = 4 * (idx % C4);
@@ -636,15 +650,18 @@ static int attention_entry(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, con
                            int flags) {
   if (!Q || !K || !Vt || !O || !strides || !lut || (keep && (!S || !P)))
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: null pointer");
-  if (!(flags & ANVIL_OP_UNCHECKED) || (flags & ~(ANVIL_OP_UNCHECKED | ANVIL_ATTN_S24 | ANVIL_ATTN_V_ROWS)))
+  if (!(flags & ANVIL_OP_UNCHECKED) || (flags & ~(ANVIL_OP_UNCHECKED | ANVIL_ATTN_S24 | ANVIL_ATTN_V_ROWS | ANVIL_ATTN_RAGGED)))
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: flags must hold ANVIL_OP_UNCHECKED (a proven graph)");
   const bool vrows = flags & ANVIL_ATTN_V_ROWS;
-  if (vrows && T != 16) return set_error(ANVIL_E_VALUE, "anvil_attention_i8: ANVIL_ATTN_V_ROWS needs T = 16");
-  if (batch0 < 1 || batch1 < 1 || (T != 16 && (T < 32 || T % 32 || T > 1024)))
+  if (vrows && (T != 16 || D > 32)) return set_error(ANVIL_E_VALUE, "anvil_attention_i8: ANVIL_ATTN_V_ROWS needs T = 16");
+  // ANVIL_ATTN_RAGGED admits any T up to 1024 (and any head dim at T = 16); T = 16 with D up to 32 keeps its kernel
+  const bool ragged = flags & ANVIL_ATTN_RAGGED;
+  const bool t16 = T == 16 && D <= 32;
+  if (batch0 < 1 || batch1 < 1 || T < 1 || T > 1024 || (!ragged && T != 16 && T % 32))
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: T=%d must be 16 or a multiple of 32 in [32, 1024]", T);
   if (D != 16 && D != 32 && D != 64 && D != 128)
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: head dim %d not in {16, 32, 64, 128}", D);
-  if (T == 16 && D > 32)
+  if (T == 16 && D > 32 && !ragged)
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: T=16 takes head dims 16 and 32, not %d", D);
   if (s_s < 0 || s_s > 31 || s_o < 0 || s_o > 31) return set_error(ANVIL_E_VALUE, "shift outside [0, 31]");
   if (one < 1 || one > 127) return set_error(ANVIL_E_VALUE, "one=%d does not fit int8", one);
@@ -657,11 +674,11 @@ static int attention_entry(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, con
                        (long long)st[i], i < 9 ? 16 : 4);
   if (!al(Q, 16) || !al(K, 16) || !al(Vt, 16) || !al(O, 4))
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: operand not aligned");
-  if ((long long)batch0 * batch1 * std::max(1, T / 32) > (1ll << 31) - 1)
+  if ((long long)batch0 * batch1 * ((T + 31) / 32) > (1ll << 31) - 1)
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: too many heads");
   // K and V^T are read through 32-bit buffer offsets over one head: T key rows of stride ldk (each at least D
   // bytes apart), D rows of V^T of stride ldv (each at least T keys)
-  if (st[5] < D || st[8] < (vrows ? D : T) || (long long)T * st[5] >= (1ll << 31) ||
+  if (st[5] < D || st[8] < (vrows ? D : T) || (t16 ? T : (T + 31ll) / 32 * 32) * st[5] >= (1ll << 31) ||
       (long long)(vrows ? T : D) * st[8] >= (1ll << 31))
     return set_error(ANVIL_E_VALUE, "anvil_attention_i8: K row stride %lld / V^T row stride %lld out of range",
                      (long long)st[5], (long long)st[8]);
@@ -672,7 +689,8 @@ static int attention_entry(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, con
       if (st[i] < 0 || st[i] % 16)
         return set_error(ANVIL_E_VALUE, "anvil_attention_i8_keep: stride %d (%lld) not a multiple of 16", i,
                          (long long)st[i]);
-    if (st[14] < T || st[17] < T || 32 * st[14] >= (1ll << 31) || 32 * st[17] >= (1ll << 31))
+    const int tw = t16 ? T : (T + 31) / 32 * 32;   // whole 32-key tiles are stored
+    if (st[14] < tw || st[17] < tw || 32 * st[14] >= (1ll << 31) || 32 * st[17] >= (1ll << 31))
       return set_error(ANVIL_E_VALUE, "anvil_attention_i8_keep: S / P row stride %lld / %lld out of range",
                        (long long)st[14], (long long)st[17]);
     if (!al(S, 16) || !al(P, 16)) return set_error(ANVIL_E_VALUE, "anvil_attention_i8_keep: S or P not aligned");
@@ -700,8 +718,8 @@ static int attention_entry(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, con
   a.clo_o = (int)std::max(-128ll * (1ll << s_o), I32_MIN);
   a.chi_o = (int)std::min(128ll * (1ll << s_o) - 1, I32_MAX);
   a.ldo32 = (int)st[11];
-  a.obytes = (int)(31 * st[11] + D);
-  a.nqt = T / 32;
+  a.masked = causal || T % 32;
+  a.nqt = (T + 31) / 32;
   auto magic = [](int d, unsigned long long& m, int& k) {
     k = 0;
     while ((1 << k) < d) ++k;
@@ -717,13 +735,12 @@ static int attention_entry(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, con
     a.sc0 = st[12], a.sc1 = st[13], a.ldsc = st[14];
     a.pr0 = st[15], a.pr1 = st[16], a.ldpr = st[17];
     a.ldsc32 = (int)st[14], a.ldpr32 = (int)st[17];
-    a.scbytes = (int)(31 * st[14] + T), a.prbytes = (int)(31 * st[17] + T);
   } else {
     a.sc0 = a.sc1 = a.ldsc = a.pr0 = a.pr1 = a.ldpr = 0;
-    a.ldsc32 = a.ldpr32 = a.scbytes = a.prbytes = 0;
+    a.ldsc32 = a.ldpr32 = 0;
   }
   const bool s24 = flags & ANVIL_ATTN_S24;
-  if (T == 16) {
+  if (t16) {
     const long long nh = (long long)batch0 * batch1;
     if (keep)
       s24 ? launch_attention_t16<true, true>(a, D, nh, ctx->stream) : launch_attention_t16<false, true>(a, D, nh, ctx->stream);

@@ -276,8 +276,10 @@ int anvil_softmax_lut_ex(anvil_ctx* ctx, const int8_t* x, const int32_t* lut, in
  * T may also be 16, with D 16 or 32 (one lane a query row); then ANVIL_ATTN_V_ROWS passes V itself, (T, D) rows of
  * stride ldv >= D, in place of V^T.
  * flags must hold ANVIL_OP_UNCHECKED: the caller has proven every int32 intermediate of the three ops in range;
- * ANVIL_ATTN_S24 adds that every |Q K^T| and |m_s| is below 2^23 (the score requant multiply is then 24-bit). */
-enum anvil_attn_flags { ANVIL_ATTN_S24 = 2, ANVIL_ATTN_V_ROWS = 4 };
+ * ANVIL_ATTN_S24 adds that every |Q K^T| and |m_s| is below 2^23 (the score requant multiply is then 24-bit);
+ * ANVIL_ATTN_RAGGED admits any T in [1, 1024] (and any of the head dims at T = 16): the bytes of V^T's rows from T up to
+ * the next multiple of 32 may hold anything. */
+enum anvil_attn_flags { ANVIL_ATTN_S24 = 2, ANVIL_ATTN_V_ROWS = 4, ANVIL_ATTN_RAGGED = 8 };
 int anvil_attention_i8(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, const int8_t* Vt, int8_t* O, int batch0,
                        int batch1, int T, int D, const int64_t* strides, int32_t m_s, int s_s, const int32_t* lut,
                        int32_t one, int causal, int32_t m_o, int s_o, int flags);
@@ -287,7 +289,8 @@ int anvil_attention_i8(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, const i
  * among them): anvil_attention_i8, which also stores the whole T x T int8 score matrix into S and the probabilities
  * into P (0 for masked keys), per (b0, b1). strides = the twelve of anvil_attention_i8, then {ss0, ss1, lds} of S
  * and {sp0, sp1, ldp} of P, all multiples of 16, with lds, ldp >= T and 32 * lds, 32 * ldp below 2^31; S and P
- * 16-byte aligned. Same preconditions and flags. */
+ * 16-byte aligned. Same preconditions and flags; with ANVIL_ATTN_RAGGED, lds and ldp are at least T rounded up to a
+ * multiple of 32 (16 at T = 16 with D up to 32), and the bytes of each row from T up to there are written too. */
 int anvil_attention_i8_keep(anvil_ctx* ctx, const int8_t* Q, const int8_t* K, const int8_t* Vt, int8_t* O, int8_t* S,
                             int8_t* P, int batch0, int batch1, int T, int D, const int64_t* strides, int32_t m_s,
                             int s_s, const int32_t* lut, int32_t one, int causal, int32_t m_o, int s_o, int flags);
