@@ -42,7 +42,6 @@
 
 namespace anvil {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 struct AttnArgs {

@@ -115,6 +115,18 @@ __device__ __forceinline__ unsigned pack4(int v0, int v1, int v2, int v3) {
   return __builtin_amdgcn_perm(t23, t01, 0x05040100u);
 }
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v4i pack16(const int* v) {   // 16 results as int8
+  return v4i{(int)pack4(v[0], v[1], v[2], v[3]), (int)pack4(v[4], v[5], v[6], v[7]), (int)pack4(v[8], v[9], v[10], v[11]),
+             (int)pack4(v[12], v[13], v[14], v[15])};
+}
+__device__ __forceinline__ v4i pack8h(const int* v) {   // 8 results as int16
+  v4i w;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) w[q] = (int)__builtin_amdgcn_perm((unsigned)v[2 * q + 1], (unsigned)v[2 * q], 0x05040100u);
+  return w;
+}
+
 constexpr unsigned RSRC_DW3 = 0x00020000u;               // raw buffer, 32-bit data format (gfx9 family)
 constexpr unsigned OOB = 0xFFFFFFF0u;                    // a buffer offset past any descriptor's range: loads 0
 
@@ -243,6 +255,37 @@ __device__ __forceinline__ int mul_sbytes(unsigned x, unsigned w) {
   else
     asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3 src1_sel:BYTE_3"
         : "=v"(d) : "v"(x), "v"(w));
+  return d;
+}
+
+template <int H, int B>
+__device__ __forceinline__ int mul_half_byte(unsigned x, unsigned w) {   // sext(half H of x) * sext(byte B of w)
+  int d;
+  if constexpr (H == 0 && B == 0)
+    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:BYTE_0"
+        : "=v"(d) : "v"(x), "v"(w));
+  else if constexpr (H == 1 && B == 1)
+    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:BYTE_1"
+        : "=v"(d) : "v"(x), "v"(w));
+  else if constexpr (H == 0 && B == 2)
+    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:BYTE_2"
+        : "=v"(d) : "v"(x), "v"(w));
+  else
+    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:BYTE_3"
+        : "=v"(d) : "v"(x), "v"(w));
+  static_assert((H == 0 && (B == 0 || B == 2)) || (H == 1 && (B == 1 || B == 3)), "entry 2q + H sits in byte B");
+  return d;
+}
+
+template <int H>
+__device__ __forceinline__ int square_half(unsigned x) {                 // sext(half H of x)^2
+  int d;
+  if constexpr (H == 0)
+    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_0"
+        : "=v"(d) : "v"(x));
+  else
+    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_1"
+        : "=v"(d) : "v"(x));
   return d;
 }
 

@@ -1,0 +1,278 @@
+// What the GEMM kernels (gemm.hip, gemm_deep.hip) share: their arguments, LDS swizzle, direct-to-LDS loads, waits, and the
+// register epilogue.
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+
+namespace anvil {
+
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+struct GemmArgs {
+  const int8_t* A;
+  const int8_t* B;
+  void* C;
+  int M, N, K;
+  int batch1;
+  int tiles_m, tiles_n;
+  long long sa0, sa1, lda, sb0, sb1, ldb, sc0, sc1, ldc;
+  // bytes from one 64-byte K block of an operand row to the next: 64 for row-major operands; for K-blocked ones
+  // (fast kernels only) the block stride, with lda / ldb then 64 (row r's block j at r 64 + j kba)
+  long long kba, kbb;
+  long long kbc;        // the same for the result's 64-column blocks (64: row-major; fast kernels only otherwise)
+  int mult, shift, rnd;
+  const int8_t* lut;
+  unsigned* flags;
+  int causal;
+  int vec_store;
+  // fused residual add (fast kernel only): D = clamp_i8((R ma + y mb + rnd2) >> shift2), y written when store_y
+  const int8_t* R;
+  int8_t* D;
+  long long sr0, sr1, ldr, sd0, sd1, ldd;
+  int ma, mb, shift2, rnd2;
+  int res, store_y, vec_res;
+  int nbatch;                     // batch0 * batch1 (persistent kernel)
+  // split-K (fast kernel, batch 1): workgroup (tile, z) stores the int32 sums of K bytes [z kchunk, (z + 1) kchunk)
+  // as partial tile (tile, z) of ws; splitk_reduce adds the partial tiles up
+  int* ws;
+  int kchunk, splits;
+  // fused rmsnorm of D (gemm_i8_fast with NORM, one tile spanning D's rows): H = rmsnorm_int(D, nw, nlut, nmult,
+  // nshift), H row-major (row stride ldh) or K-blocked (block stride kbh); nbits = the bit length of nlut_len
+  const int8_t* nw;
+  const int* nlut;
+  int8_t* H;
+  long long ldh, kbh;
+  int nlut_len, nbits, nmult, nshift;
+};
+
+constexpr int G_THREADS = 256;
+constexpr int GROUP_M = 4;
+
+// Element offset of result (m, n) from the batch entry's base: row-major (kbc = 64) or K-blocked (ldc = 64, column
+// block n / 64 at kbc). A 16-byte store chunk never crosses a 64-column block.
+__device__ __forceinline__ long long cpos(const GemmArgs& g, int m, int n) {
+  return (long long)m * g.ldc + (long long)(n >> 6) * g.kbc + (n & 63);
+}
+
+// Bytes of a tile's operand rows that its buffer descriptor covers: rows whole rows of a row-major operand (kb = 64),
+// or, K-blocked, those rows in every K block; anything past reads as zero.
+__device__ __forceinline__ int operand_bytes(int rows, long long ld, long long kb, int K) {
+  // row-major: up to the last row's K-th byte, not its row stride: an operand that is a column slice of a wider
+  // array (one head of q, say) must not reach past that array's last row, where its allocation may end
+  return kb == 64 ? (int)((rows - 1) * ld + K) : (int)(rows * 64 + ((K + 63) / 64 - 1) * kb);
+}
+
+// Physical 16-byte chunk of logical chunk `chunk` in LDS row `row`. gfx950's LDS serves a ds_read_b128 from 64
+// banks (256 bytes a cycle) to 16 lanes at a time, taken as four blocks of four consecutive lanes whose block
+// indices k differ in the pattern {0, 3, 5, 6} (+ 8 m, and the complementary {1, 2, 4, 7}); measured on MI355X with
+// a read-pattern probe. A fragment read puts rows 4 k + j (j = 0..3) of one logical chunk in block k, so the
+// swizzle must differ for k = 0, 3, 5, 6 at each j: chunk ^ ((row ^ row >> 2) & 3) = chunk ^ ((j ^ k) & 3) does, and
+// reads at 195 B/clk/CU against 108 for the 2-way-conflicting ((row >> 1) ^ (row >> 3)) & 3.
+template <int BK>
+__device__ __forceinline__ int swz(int row, int chunk) {
+  static_assert(BK == 64 || BK == 128, "swizzle defined for 64- and 128-byte rows");
+  if (BK == 64) return chunk ^ ((row ^ (row >> 2)) & 3);
+  return chunk ^ ((row ^ (row >> 3)) & 7);
+}
+
+// 16 bytes per lane from buffer offset voff into LDS at lds + 16 * lane (lds must be wave-uniform)
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, int8_t* lds, unsigned voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
+}
+
+__device__ __forceinline__ void wait_vmcnt(int n) {
+  // s_waitcnt with vmcnt = n (0..15), expcnt and lgkmcnt left at their "no wait" maxima
+  switch (n) {
+    case 0: __builtin_amdgcn_s_waitcnt(0x0F70); break;
+    case 1: __builtin_amdgcn_s_waitcnt(0x0F71); break;
+    case 2: __builtin_amdgcn_s_waitcnt(0x0F72); break;
+    case 3: __builtin_amdgcn_s_waitcnt(0x0F73); break;
+    case 4: __builtin_amdgcn_s_waitcnt(0x0F74); break;
+    case 5: __builtin_amdgcn_s_waitcnt(0x0F75); break;
+    case 6: __builtin_amdgcn_s_waitcnt(0x0F76); break;
+    case 7: __builtin_amdgcn_s_waitcnt(0x0F77); break;
+    case 8: __builtin_amdgcn_s_waitcnt(0x0F78); break;
+    case 10: __builtin_amdgcn_s_waitcnt(0x0F7A); break;
+    case 12: __builtin_amdgcn_s_waitcnt(0x0F7C); break;
+    default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
+  }
+}
+
+// all waves' LDS writes for a stage have landed once each has waited for its own loads and the barrier is passed;
+// the acquire fence keeps the following LDS reads below the barrier without waiting on later loads
+__device__ __forceinline__ void stage_barrier() {
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// s_waitcnt vmcnt(N) lgkmcnt(0): this wave's loads beyond the newest N have landed and its LDS accesses are done
+template <int N>
+__device__ __forceinline__ void wait_vm_lgkm0() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0070);
+}
+
+// (x >> sh) & 255 by one SDWA shift (byte 0 written, the rest zeroed): the LUT index of a clamped int8 result
+__device__ __forceinline__ unsigned sra_byte(int x, int sh) {
+  unsigned d;
+  asm("v_ashrrev_i32_sdwa %0, %1, %2 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:DWORD"
+      : "=v"(d) : "s"(sh), "v"(x));
+  return d;
+}
+
+// requant (+ LUT) of one lane's 16 accumulators into 16 results. With the rotated LUT (LUT 1: int8 results, the
+// table staged so that the entry of v sits at index v & 255) the clamp runs before the shift, with bounds
+// [-128, 127] << shift saturated to int32, and one SDWA shift gives the lookup index. The widened table (LUT 2, entry
+// u = lut[clamp(u - 2^(31 - shift), -128, 127) + 128]) is indexed by (x + 2^31) >> shift, unsigned.
+template <int OSZ, bool MUL24, int LUT>
+__device__ __forceinline__ void requant16(const v16i& a, int mult, int rnd, int shift, const int8_t* lut_s, int v[16]) {
+  if constexpr (LUT == 2) {
+    static_assert(OSZ == 1, "a LUT epilogue has int8 results");
+    const unsigned rndw = (unsigned)rnd ^ 0x80000000u;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const unsigned u = (unsigned)(MUL24 ? __mul24(a[e], mult) : a[e] * mult) + rndw;
+      v[e] = lut_s[u >> shift];
+    }
+  } else if constexpr (LUT == 1) {
+    static_assert(OSZ == 1, "a LUT epilogue has int8 results");
+    const int clo = (int)max(-128ll << shift, (long long)INT32_MIN);
+    const int chi = (int)min((128ll << shift) - 1, (long long)INT32_MAX);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int x = MUL24 ? (__mul24(a[e], mult) + rnd) : (a[e] * mult + rnd);
+      v[e] = lut_s[sra_byte(med3i(x, clo, chi), shift)];
+    }
+  } else {
+    const int lo = OSZ == 1 ? -128 : -32768, hi = OSZ == 1 ? 127 : 32767;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int x = MUL24 ? (__mul24(a[e], mult) + rnd) : (a[e] * mult + rnd);
+      v[e] = min(max(x >> shift, lo), hi);
+    }
+  }
+}
+
+
+// Epilogue from registers: tile (i, j) of this lane is row mrow + 32 j, columns ncol + 32 i .. + 15. Interior tiles
+// issue every residual load first, then requantize and store 16 bytes a lane; edge tiles store element by element.
+template <int BM, int BN, int WM, int WN, int TM, int TN, int OSZ, bool MUL24>
+__device__ __forceinline__ void direct_epilogue(const GemmArgs& g, const v16i (&acc)[TN][TM], const int8_t* lut_s,
+                                                bool wide, int mrow, int ncol, int m0, int n0, int b0, int b1) {
+  char* Cb = reinterpret_cast<char*>(g.C) + (b0 * g.sc0 + b1 * g.sc1) * OSZ;
+  const bool res = OSZ == 1 && g.res;
+  const int8_t* Rb = g.R + b0 * g.sr0 + b1 * g.sr1;
+  int8_t* Db = g.D + b0 * g.sd0 + b1 * g.sd1;
+  const bool interior = m0 + BM <= g.M && n0 + BN <= g.N &&
+                        (res ? (g.vec_res != 0 && (!g.store_y || g.vec_store != 0)) : g.vec_store != 0);
+  const int mult = g.mult, rnd = g.rnd, shift = g.shift;
+  auto run = [&](auto lut_c, auto full_c) {
+    constexpr int LUT = decltype(lut_c)::value;
+    constexpr bool FULL = decltype(full_c)::value;
+    v4i rv[TM][TN];
+    if (FULL && res) {
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+          rv[j][i] = *reinterpret_cast<const v4i*>(Rb + (long long)(mrow + 32 * j) * g.ldr + ncol + 32 * i);
+    }
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int m = mrow + 32 * j;
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        const int n = ncol + 32 * i;
+        int v[16];
+        requant16<OSZ, MUL24, LUT>(acc[i][j], mult, rnd, shift, lut_s, v);
+        if (FULL) {
+          if (res) {
+            const int ma = g.ma, mb = g.mb, rnd2 = g.rnd2, sh2 = g.shift2;
+            v4i ov;
+            if (PackedAdd::applies(ma, mb)) {
+              // multipliers below 2^24: y packed, then full-rate byte multiplies (PackedAdd)
+              const PackedAdd add(ma, mb, rnd2, sh2);
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                ov[q] = (int)add((unsigned)rv[j][i][q], pack4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]));
+            } else {
+              // clamp before the shift, then one SDWA shift into each byte lane
+              const int clo2 = (int)max(-128ll << sh2, (long long)INT32_MIN);
+              const int chi2 = (int)min((128ll << sh2) - 1, (long long)INT32_MAX);
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                int o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const int r = (int)(int8_t)((unsigned)rv[j][i][q] >> (8 * e));
+                  o[e] = med3i(r * ma + v[4 * q + e] * mb + rnd2, clo2, chi2);   // proven inside int32
+                }
+                ov[q] = (int)sra_pack4(o[0], o[1], o[2], o[3], sh2);
+              }
+            }
+            *reinterpret_cast<v4i*>(Db + (long long)m * g.ldd + n) = ov;
+            if (!g.store_y) continue;
+          }
+          if (OSZ == 1) {
+            v4i w;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w[q] = (int)pack4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+            *reinterpret_cast<v4i*>(Cb + cpos(g, m, n)) = w;
+          } else {
+            v4i w0, w1;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              w0[q] = (int)__builtin_amdgcn_perm((unsigned)v[2 * q + 1], (unsigned)v[2 * q], 0x05040100u);
+              w1[q] = (int)__builtin_amdgcn_perm((unsigned)v[2 * q + 9], (unsigned)v[2 * q + 8], 0x05040100u);
+            }
+            char* d = Cb + cpos(g, m, n) * 2;
+            *reinterpret_cast<v4i*>(d) = w0;
+            *reinterpret_cast<v4i*>(d + 16) = w1;
+          }
+        } else if (m < g.M) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            if (n + e >= g.N) break;
+            if (res) {
+              const int r = Rb[(long long)m * g.ldr + n + e];
+              Db[(long long)m * g.ldd + n + e] =
+                  (int8_t)min(max((r * g.ma + v[e] * g.mb + g.rnd2) >> g.shift2, -128), 127);
+              if (!g.store_y) continue;
+            }
+            if (OSZ == 1)
+              Cb[cpos(g, m, n) + e] = (int8_t)v[e];
+            else
+              reinterpret_cast<int16_t*>(Cb)[cpos(g, m, n) + e] = (int16_t)v[e];
+          }
+        }
+      }
+    }
+  };
+  const bool lut = OSZ == 1 && g.lut;
+  auto pick = [&](auto full_c) {
+    if constexpr (OSZ == 1) {
+      if (lut && wide) return run(std::integral_constant<int, 2>{}, full_c);
+      if (lut) return run(std::integral_constant<int, 1>{}, full_c);
+    }
+    run(std::integral_constant<int, 0>{}, full_c);
+  };
+  if (interior) pick(std::true_type{}); else pick(std::false_type{});
+}
+
+static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// the products of one grouped launch: member i owns the workgroups [first[i], first[i + 1])
+constexpr int GEMM_GROUP_MAX = 4;
+struct GemmGroupArgs {
+  GemmArgs g[GEMM_GROUP_MAX];
+  int first[GEMM_GROUP_MAX + 1];
+  int n;
+};
+
+// gemm_deep.hip: a product, or a group of them, on 64 x 64 tiles with ns (2 or 4) stages of 128 K bytes
+void launch_deep(GemmArgs& g, int ns, int osz, bool mul24, int batch, hipStream_t s);
+void launch_deep_group(GemmArgs* gs, const int* batch, int n, int ns, int osz, bool mul24, hipStream_t s);
+
+}  // namespace anvil

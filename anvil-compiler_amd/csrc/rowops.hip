@@ -47,7 +47,6 @@ __device__ __forceinline__ int wave_sum32(int v) {
   return v;
 }
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ int sbyte(const v4i& v, int b) {   // signed byte b (0..15) of a 16-byte chunk
@@ -445,37 +444,6 @@ __global__ __launch_bounds__(R_THREADS) void rmsnorm_narrow(const int8_t* __rest
 // Each entry's square is one 24-bit multiply of its sign-extended half (SDWA); x w is one 24-bit multiply of that
 // half by the sign-extended weight byte, |x w| <= 2^22. With s24 (every |lut[i] M| < 2^23) x w (lut[i] M) + rnd is one 24-bit multiply-add; without
 // it the product wraps in 32 bits, which is exact because x w lut[i] M + rnd is proven to fit int32.
-template <int H, int B>
-__device__ __forceinline__ int mul_half_byte(unsigned x, unsigned w) {   // sext(half H of x) * sext(byte B of w)
-  int d;
-  if constexpr (H == 0 && B == 0)
-    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:BYTE_0"
-        : "=v"(d) : "v"(x), "v"(w));
-  else if constexpr (H == 1 && B == 1)
-    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:BYTE_1"
-        : "=v"(d) : "v"(x), "v"(w));
-  else if constexpr (H == 0 && B == 2)
-    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:BYTE_2"
-        : "=v"(d) : "v"(x), "v"(w));
-  else
-    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:BYTE_3"
-        : "=v"(d) : "v"(x), "v"(w));
-  static_assert((H == 0 && (B == 0 || B == 2)) || (H == 1 && (B == 1 || B == 3)), "entry 2q + H sits in byte B");
-  return d;
-}
-
-template <int H>
-__device__ __forceinline__ int square_half(unsigned x) {                 // sext(half H of x)^2
-  int d;
-  if constexpr (H == 0)
-    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_0"
-        : "=v"(d) : "v"(x));
-  else
-    asm("v_mul_i32_i24_sdwa %0, sext(%1), sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_1"
-        : "=v"(d) : "v"(x));
-  return d;
-}
-
 constexpr int WIDE_LUT_MAX = 4096;                               // table words the wide kernel stages in LDS
 
 template <int L, int CH>
