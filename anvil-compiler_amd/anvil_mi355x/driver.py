@@ -24,6 +24,7 @@ import numpy as np
 from . import hostpar
 from . import ir as g
 from . import quantize as Q
+from . import rowprog
 from . import runtime as rt
 from .layout import Buf, View, contig_strides
 
@@ -182,6 +183,8 @@ class CompiledModel:
         self._const_kb = {}
         self._const_bt_host = {}
         self._plans = {}
+        self._row_streams = {}
+        self.row_programs = True          # runs of row-wise ops as one anvil_row_program launch (rowprog.py)
         self.group_gemms = True           # independent consecutive GEMMs as one anvil_gemm_i8_group call
 
     # --------------------------------------------------------------------------------------- layout choice
@@ -330,8 +333,15 @@ class CompiledModel:
         adds = self._residual_fusions(keep)
         P.norm_of = self._norm_fusions(adds)
         P.kb_values = self._kblocked_values(keep, fused, skip, adds)
+        # the runs of row-wise ops (a device without the entry point runs them op by op)
+        first = {}
+        if self.row_programs and hasattr(dev, "row_program"):
+            first = {prog.ops[0]: prog for prog in rowprog.find(self, nb)}
+        done = set()
         for op in self.ops:
-            if op in skip or op in P.fused_adds or op in P.fused_norms:
+            if op in first and rowprog.plan(self, P, first[op], views, nb, keep, step):
+                done.update(first[op].ops)
+            if op in skip or op in P.fused_adds or op in P.fused_norms or op in done:
                 continue
             r = op.results[0]
             t = g.qt(r)
@@ -577,6 +587,14 @@ class CompiledModel:
             b.mem = mem
             self._const_kb[key] = View(b, "i8", (N, K), (64, 1), kb=N * 64)
         return self._const_kb[key]
+
+    def _row_stream(self, lay):
+        """The weights of a row program's products as one device buffer (rowprog.pack_weights), kept for every plan."""
+        key = tuple(map(id, lay["stream"]))
+        if key not in self._row_streams:
+            parts = [rowprog.pack_weights(self._bt_host(self._bt_const(op))).reshape(-1) for op in lay["stream"]]
+            self._row_streams[key] = self.dev.upload(np.concatenate(parts)) if parts else None
+        return self._row_streams[key]
 
     def _bt_host(self, bt):
         """Host copy of a const operand view made by _bt_const (kept on the host when it was uploaded)."""
@@ -1210,6 +1228,8 @@ def _work(fn, args):
         _, a, bt, c, M, N, K = args[:7]
         nw, nlut = args[16], args[17]
         return "gemm", 2 * M * N * K, M * K + N * K + M * N * (4 if c is not None else 3) + N + 4 * nlut.size
+    if fn is rowprog.call:
+        return args[1].work()
     if fn is _call_attention:
         _, q, k, v, o, b0, b1, T, D = args[:9]
         nb = b0 * b1

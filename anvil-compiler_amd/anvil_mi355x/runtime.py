@@ -68,6 +68,9 @@ SIGNATURES = {
     "anvil_gemm_i8_add_ex": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _p, _i32, _i, _p, _i, _p, _i32, _i32, _i, _p, _p,
                              _i],
     "anvil_gemm_i8_add_norm": [_p, _p, _p, _p, _i, _i, _i, _p, _i32, _i, _p, _p, _i32, _i32, _i, _p, _p, _p, _i],
+    "anvil_row_create": [_p, _p, _i, _i64, _i, _p, _i64, _p, _i, C.POINTER(_p)],
+    "anvil_row_launch": [_p, _p],
+    "anvil_row_destroy": [_p, _p],
     "anvil_rmsnorm_int": [_p, _p, _i, _p, _p, _i, _i32, _i, _i, _i32, _i64, _i, _p],
     "anvil_rmsnorm_int_ex": [_p, _p, _i, _p, _p, _i, _i32, _i, _i, _i32, _i64, _i, _p, _i],
     "anvil_softmax_lut": [_p, _p, _p, _i32, _i, _i64, _i, _i, _p, _i],
@@ -98,6 +101,15 @@ class NormEpilogue(C.Structure):
     _fields_ = [("w", _p), ("lut", _p), ("lut_len", _i32), ("mult", _i32), ("shift", _i32), ("out", _p),
                 ("ld", _i64), ("kb", _i64)]
 
+
+class RowOp(C.Structure):
+    """anvil_row_op: one op of a row program."""
+    _fields_ = [(f, _i32) for f in ("kind", "a", "b", "dst", "n", "k", "table", "m24", "wide", "wide_a", "wide_b", "trans",
+                                    "mult", "mult2", "shift", "c", "e", "lut_len")] + [
+        ("in", _p), ("lut", _p), ("out", _p), ("ld", _i64), ("kb", _i64)]
+
+
+ROW_LOAD, ROW_NORM, ROW_GEMM, ROW_ADD, ROW_LUT, ROW_LUT_MUL = 1, 2, 3, 4, 5, 6
 
 GEMM_GROUP_MAX = 4
 _lib = None
@@ -222,6 +234,27 @@ class HipGraph:
     def free(self):
         if self.handle and self.dev.ctx:
             self.dev.lib.call("anvil_graph_destroy", self.dev.ctx, C.c_void_p(self.handle))
+        self.handle = 0
+
+    def __del__(self):
+        try:
+            self.free()
+        except Exception:
+            pass
+
+
+class RowProgram:
+    """A row program of a Device (anvil_row_create), run by launch(); freed when collected."""
+
+    def __init__(self, dev: "Device", handle: int):
+        self.dev, self.handle = dev, int(handle)
+
+    def launch(self):
+        self.dev.lib.call("anvil_row_launch", self.dev.ctx, self.handle)
+
+    def free(self):
+        if self.handle and self.dev.ctx:
+            self.dev.lib.call("anvil_row_destroy", self.dev.ctx, C.c_void_p(self.handle))
         self.handle = 0
 
     def __del__(self):
@@ -368,6 +401,15 @@ class Device:
                       C.c_void_p(_ptr(Cp) if Cp is not None else 0), M, N, K, st, int(mult), shift,
                       C.c_void_p(_ptr(lut) if lut is not None else 0), C.c_void_p(_ptr(R)), int(ma), int(mb), shift2,
                       C.c_void_p(_ptr(D)), rs, C.byref(norm), int(flags))
+
+    def row_program(self, ops, rows, seq, stream, tables, ntables) -> "RowProgram":
+        """anvil_row_create: a ctypes array of RowOp over `rows` rows, the weight stream (a device buffer, or None) and
+        a ctypes array of table pointers, as a callable program."""
+        handle = C.c_void_p()
+        self.lib.call("anvil_row_create", self.ctx, ops, len(ops), rows, seq,
+                      C.c_void_p(_ptr(stream) if stream is not None else 0), stream.nbytes if stream is not None else 0,
+                      tables, ntables, C.byref(handle))
+        return RowProgram(self, handle.value)
 
     def rmsnorm_int(self, x, x_dtype, w, lut, lut_len, mult, shift, ss_shift, ss_init, rows, cols, out, flags=0):
         self.lib.call("anvil_rmsnorm_int_ex", self.ctx, C.c_void_p(_ptr(x)), DTYPE_CODE[x_dtype], C.c_void_p(_ptr(w)),

@@ -227,6 +227,53 @@ int anvil_gemm_i8_add_ex(anvil_ctx* ctx, const int8_t* A, const int8_t* Bt, void
                          const void* R, int32_t ma, int32_t mb, int shift2, void* D, const int64_t* rstrides,
                          int flags);
 
+/* Row programs: a run of row-wise ops of a proven graph over the rows of one activation, in one launch (the reference
+ * evaluates them op by op, anvil/interp/graph.py:62-75). A value lives in LDS, in slots of one KiB (32 rows of 32 columns):
+ * ceil(n / 32) of them at int8 and twice as many at int16, from slot a, b or dst on. The LOADs come first.
+ *   LOAD     dst = rows of `in` (ld, kb as below)
+ *   NORM     dst = rmsnorm_int(a) (anvil/semantics.py:164-182): weights `in` (n int8), table lut (lut_len int32 >= 0, a
+ *            multiple of 4 up to 4096), mult, shift, square shift c, start value e; |x w| and |lut[i] * mult| below 2^23
+ *   GEMM     dst = requant(a @ W) [-> table] (:95-103), k blocks of 32 K bytes of a, its weights next in the stream; m24:
+ *            |acc| and |mult| below 2^23. trans: the int8 result goes to `out` only, transposed per sequence: row
+ *            r = b * seq + t, column j at out + b * kb + j * ld + t
+ *   ADD      dst = add_requant(a * mult + b * mult2) (:106-115); m24: multipliers below 2^24 (int8 throughout) or 2^23
+ *   LUT      dst = table[a] (:87-92);  LUT_MUL  dst = requant(table[a] * b, mult, shift); m24: |mult| below 2^23
+ * wide, wide_a, wide_b: dst (LOAD: the input), a, b are int16. Every result is also written to `out` unless NULL, at
+ * row r, column j: out + r * ld + (j / 64) * kb + j % 64 at int8 (kb = 64: row-major, else K-blocked, ld = 64), r * ld + j
+ * at int16. An element-wise op's dst may be the slot of an operand of its own size. Widths n are multiples of 16; every
+ * int32 intermediate is proven in range (as ANVIL_OP_UNCHECKED states). The weight stream w holds each GEMM's weights in
+ * op order, zero-padded to whole blocks, [n / 32][k] fragments of 64 lanes x 16 bytes: lane l holds K bytes
+ * 32 k + 16 (l / 32) .. + 15 of weight row (result column) 32 nb + 16 ((i >> 2) & 1) + 4 (i >> 3) + (i & 3), i = l % 32. The
+ * stream, the tables and one wave's slots together fit in 96 KiB. */
+enum anvil_row_kind {
+  ANVIL_ROW_LOAD = 1,
+  ANVIL_ROW_NORM = 2,
+  ANVIL_ROW_GEMM = 3,
+  ANVIL_ROW_ADD = 4,
+  ANVIL_ROW_LUT = 5,
+  ANVIL_ROW_LUT_MUL = 6
+};
+enum { ANVIL_ROW_OPS_MAX = 24, ANVIL_ROW_TABLES_MAX = 4, ANVIL_ROW_SLOTS_MAX = 64 };
+typedef struct anvil_row_op {
+  int32_t kind, a, b, dst;
+  int32_t n, k, table, m24;          /* table: index into `tables`, -1 none */
+  int32_t wide, wide_a, wide_b, trans;
+  int32_t mult, mult2, shift, c;
+  int32_t e, lut_len;
+  const void* in;
+  const int32_t* lut;
+  void* out;
+  int64_t ld, kb;
+} anvil_row_op;
+/* anvil_row_create checks a program over `rows` rows (a multiple of seq) and keeps its ops in device memory (it
+ * allocates: not inside a capture); anvil_row_launch runs it on the context's stream; anvil_row_destroy waits for the
+ * stream and frees it. Buffers and tables are the caller's and outlive the program. */
+typedef struct anvil_row_prog anvil_row_prog;
+int anvil_row_create(anvil_ctx* ctx, const anvil_row_op* ops, int nops, int64_t rows, int seq, const int8_t* w,
+                     int64_t w_bytes, const int8_t* const* tables, int ntables, anvil_row_prog** prog);
+int anvil_row_launch(anvil_ctx* ctx, anvil_row_prog* prog);
+int anvil_row_destroy(anvil_ctx* ctx, anvil_row_prog* prog);
+
 /* rmsnorm_int over rows of `cols` elements (reference anvil/semantics.py:158-182, golden.rmsnorm_int):
  *   ss = ss_init + sum_j ((x_j^2 + 2^(ss_shift-1)) >> ss_shift); (i, k) = rsqrt_index(ss, lut_len);
  *   out_j = clamp_i8((x_j * w_j * lut[i] * mult + 2^(shift+k-1)) >> (shift + k)).

@@ -1,0 +1,187 @@
+"""Row programs (anvil_row_create): the planner's runs of row-wise ops on a CPU stand-in that decodes the weight stream
+lane by lane, and the kernels against the oracle at tile edges, widths and sequence lengths where they can go wrong."""
+import gzip
+import json
+import math
+
+import numpy as np
+import pytest
+
+import anvil_mi355x
+import fake_device
+import helpers
+from anvil_mi355x import models, rowprog
+from anvil_mi355x import runtime as rt
+from oracle import interp
+from oracle import semantics as sem
+
+
+class RowFakeProgram:
+    def __init__(self, dev, args):
+        self.dev, self.args = dev, args
+
+    def launch(self):
+        self.dev.run_row_program(*self.args)
+
+
+class RowFake(fake_device.FakeDevice):
+    """The stand-in with anvil_row_program, op by op on the oracle, from the C structs."""
+
+    def row_program(self, *args):
+        return RowFakeProgram(self, args)
+
+    def run_row_program(self, ops, rows, seq, stream, tables, ntables):
+        self.calls.append(("row_program", rows, seq, len(ops)))
+        nb = 32
+        left = self._raw(stream, np.int8, stream.nbytes) if stream is not None else np.zeros(0, np.int8)
+        tabs = [self.view(tables[i], "i8", (256,), (1,)).astype(np.int64) for i in range(ntables)]
+        slots = {}
+
+        def put(o, v):
+            dt = "i16" if o.wide else "i8"
+            n = -(-o.n // nb) * (1 + o.wide)
+            assert o.dst >= 0 and o.dst + n <= rowprog.SLOTS_MAX
+            for k in [k for k, (m, _) in slots.items() if k < o.dst + n and o.dst < k + m]:
+                del slots[k]                              # overwritten
+            slots[o.dst] = (n, v)
+            if o.out and not o.trans:
+                if o.wide or o.kb == 64:
+                    self.store(o.out, dt, (rows, o.n), (o.ld, 1), v)
+                else:
+                    self.store(o.out, dt, (rows, -(-o.n // 64), 64), (64, o.kb, 1), v.reshape(rows, -1, 64))
+
+        for o in ops:
+            a = slots[o.a][1] if o.kind != rt.ROW_LOAD else None
+            if o.kind == rt.ROW_LOAD:
+                src = getattr(o, "in")
+                if o.wide or o.kb == 64:
+                    put(o, self.view(src, "i16" if o.wide else "i8", (rows, o.n), (o.ld, 1)).astype(np.int64))
+                else:
+                    v = self.view(src, "i8", (rows, o.n // 64, 64), (64, o.kb, 1)).astype(np.int64)
+                    put(o, v.reshape(rows, o.n))
+            elif o.kind == rt.ROW_NORM:
+                w = self.view(getattr(o, "in"), "i8", (o.n,), (1,)).astype(np.int64)
+                lut = self.view(o.lut, "i32", (o.lut_len,), (1,)).astype(np.int64)
+                put(o, sem.rmsnorm_wide(a, w, lut, o.mult, o.shift, o.c, o.e, "i16" if o.wide_a else "i8"))
+            elif o.kind == rt.ROW_GEMM:
+                K, N = o.k * nb, -(-o.n // nb) * nb
+                W = np.zeros((N, K), np.int64)
+                for j in range(N // nb):
+                    for k in range(o.k):
+                        frag, left = left[:1024].reshape(64, 16), left[1024:]
+                        for lane in range(64):
+                            i = lane % 32
+                            col = 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3)
+                            W[32 * j + col, 32 * k + 16 * (lane // 32):32 * k + 16 * (lane // 32) + 16] = frag[lane]
+                x = np.zeros((rows, K), np.int64)
+                x[:, :a.shape[1]] = a
+                y = sem.qmatmul(x, W.T, o.mult, o.shift, tabs[o.table] if o.table >= 0 else None,
+                                "i16" if o.wide else "i8")[:, :o.n]
+                if o.trans:
+                    self.store(o.out, "i8", (rows // seq, o.n, seq), (o.kb, o.ld, 1),
+                               y.reshape(-1, seq, o.n).transpose(0, 2, 1))
+                else:
+                    put(o, y)
+            elif o.kind == rt.ROW_ADD:
+                put(o, sem.add_requant(a, slots[o.b][1], o.mult, o.mult2, o.shift, "i16" if o.wide else "i8"))
+            elif o.kind == rt.ROW_LUT:
+                put(o, sem.lut_i8(a, tabs[o.table]))
+            else:
+                put(o, sem.swiglu_lut(a, slots[o.b][1], tabs[o.table], o.mult, o.shift))
+        assert left.size == 0
+
+
+def frozen(model):
+    with gzip.open(helpers.ROOT / "tests" / "golden" / f"model_graph_{model}.json.gz", "rt") as f:
+        body = json.load(f)
+    return anvil_mi355x.parse_ir(body["ir"]), {k: np.asarray(v, dtype=np.int64).reshape(body["shapes"][k])
+                                               for k, v in body["consts"].items()}
+
+
+def check(module, consts, model, x, keep, quantized):
+    cm = anvil_mi355x.compile(model)
+    res = cm.run(x, "mi355x", batch=True, keep=keep, quantized=quantized)
+    xq = x if quantized else cm.quantize_input(x)
+    want = interp.run(module, {cm.inputs[0]: xq}, consts, batch=True, fast=True)
+    for k in res.ints:
+        assert np.array_equal(res.ints[k], want.values[k]), (k, np.argwhere(res.ints[k] != want.values[k])[:4])
+    return cm
+
+
+def block(C, H, T, layers=1, vocab=0, gelu="fused", causal=True):
+    spec = models.BlockSpec(C, H, T, layers=layers, vocab=vocab, gelu=gelu, causal=causal, calib_batches=1)
+    return models.build(spec, 9)
+
+
+def block_inputs(built, n, seed=4):
+    return models.to_float_input(built.spec, built.params, models.eval_inputs(built.spec, n, 9, seed))
+
+
+BLOCKS = [(32, 2, 16, 1, 0, "fused"), (32, 1, 5, 2, 0, "lut"), (16, 1, 33, 1, 0, "fused"), (32, 2, 10, 2, 64, "fused"),
+          (32, 2, 7, 1, 512, "lut")]
+
+
+@pytest.mark.parametrize("C,H,T,layers,vocab,gelu", BLOCKS)
+@pytest.mark.parametrize("keep", ["outputs", "all"])
+def test_planner_runs_row_programs(monkeypatch, C, H, T, layers, vocab, gelu, keep):
+    dev = RowFake()
+    monkeypatch.setattr(rt, "device", lambda index=0: dev)
+    b = block(C, H, T, layers, vocab, gelu)
+    check(b.module, b.consts, b, block_inputs(b, 3), keep, False)
+    kinds = [c[0] for c in dev.calls if c[0] != "quantize"]
+    assert kinds == (["row_program", "attention" + ("_keep" if keep == "all" else "")] * layers + ["row_program"]
+                     + ["gemm"] * (vocab == 512))
+
+
+def test_wider_products_run_op_by_op(monkeypatch):
+    dev = RowFake()
+    monkeypatch.setattr(rt, "device", lambda index=0: dev)
+    b = block(64, 4, 8)
+    cm = check(b.module, b.consts, b, block_inputs(b, 2), "outputs", False)
+    assert "row_program" not in [c[0] for c in dev.calls]
+    assert not rowprog.find(cm, 4095) and len(rowprog.find(cm, 4096)) == 2      # 32,768 rows
+    b = block(96, 3, 8)
+    assert not rowprog.find(check(b.module, b.consts, b, block_inputs(b, 2), "outputs", False), 4096)
+
+
+@pytest.mark.parametrize("model", ["v1", "v2"])
+@pytest.mark.parametrize("keep", ["outputs", "all"])
+def test_planner_runs_the_frozen_models_as_row_programs(monkeypatch, model, keep):
+    dev = RowFake()
+    monkeypatch.setattr(rt, "device", lambda index=0: dev)
+    module, consts = frozen(model)
+    lim = 128 if model == "v1" else 1 << 15
+    check(module, consts, (module, consts), np.random.default_rng(3).integers(-lim, lim, (3, 16, 32)), keep, True)
+    assert [c[0] for c in dev.calls].count("row_program") == 3 and len(dev.calls) == 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,H,T,layers,vocab,gelu", BLOCKS)
+@pytest.mark.parametrize("nb,keep", [(1, "outputs"), (3, "all"), (37, "outputs")])
+def test_row_programs_match_the_oracle(C, H, T, layers, vocab, gelu, nb, keep):
+    """Whole blocks: widths below and at a K block (zero-padded weights), rows that end inside a tile, sequences of odd
+    length (V^T byte stores)."""
+    b = block(C, H, T, layers, vocab, gelu)
+    cm = check(b.module, b.consts, b, block_inputs(b, nb), keep, False)
+    assert any(fn is rowprog.call for _, fn, _ in cm.plan(nb, keep).steps)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,nb,keep", [(33, 993, "outputs"), (16, 2048, "all")])
+def test_64_wide_rows_match_the_oracle(T, nb, keep):
+    b = block(64, 2, T)
+    cm = check(b.module, b.consts, b, block_inputs(b, nb), keep, False)
+    assert any(fn is rowprog.call for _, fn, _ in cm.plan(nb, keep).steps)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["v1", "v2"])
+@pytest.mark.parametrize("nb", [1, 5, 700])
+@pytest.mark.parametrize("keep", ["outputs", "all"])
+def test_frozen_models_match_the_oracle(model, nb, keep):
+    module, consts = frozen(model)
+    lim = 128 if model == "v1" else 1 << 15
+    x = np.random.default_rng(nb).integers(-lim, lim, (nb, 16, 32))
+    x[0] = -lim
+    cm = check(module, consts, (module, consts), x, keep, True)
+    assert math.prod(cm.meta[cm.inputs[0]][1]) == 512
