@@ -1,4 +1,4 @@
-// What the GEMM kernels (gemm.hip, gemm_deep.hip) share: their arguments, LDS swizzle, direct-to-LDS loads, waits, and the
+// What the GEMM kernels (gemm.hip, gemm_deep.hip, gemm_any.hip) share: their arguments, LDS swizzle, direct-to-LDS loads, waits, and the
 // register epilogue.
 #pragma once
 
@@ -80,6 +80,22 @@ __device__ __forceinline__ int swz(int row, int chunk) {
 // 16 bytes per lane from buffer offset voff into LDS at lds + 16 * lane (lds must be wave-uniform)
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, int8_t* lds, unsigned voff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
+}
+
+// K bytes k .. k + 15 (k a multiple of 16) of a row of K bytes at any alignment, zeros past its end. A row's last, partial
+// chunk comes from its last 16 bytes, shifted down, so no load leaves the row.
+__device__ __forceinline__ v4i row_chunk(const int8_t* row, int k, int K) {
+  v4i v = {0, 0, 0, 0};
+  if (K >= 16) {
+    unsigned __int128 w;
+    __builtin_memcpy(&w, row + min(k, K - 16), 16);
+    const int past = k + 16 - K;                         // bytes of the chunk past the row
+    w = past >= 16 ? 0 : w >> 8 * max(past, 0);
+    __builtin_memcpy(&v, &w, 16);
+  } else {
+    for (int i = 0; k + i < K; ++i) v[i >> 2] |= (int)((unsigned)(uint8_t)row[k + i] << (8 * (i & 3)));
+  }
+  return v;
 }
 
 __device__ __forceinline__ void wait_vmcnt(int n) {
@@ -274,5 +290,8 @@ struct GemmGroupArgs {
 // gemm_deep.hip: a product, or a group of them, on 64 x 64 tiles with ns (2 or 4) stages of 128 K bytes
 void launch_deep(GemmArgs& g, int ns, int osz, bool mul24, int batch, hipStream_t s);
 void launch_deep_group(GemmArgs* gs, const int* batch, int n, int ns, int osz, bool mul24, hipStream_t s);
+
+// gemm_any.hip: a proven product of operands at any alignment and stride
+void launch_any(GemmArgs& g, int osz, bool mul24, int batch, int num_cu, hipStream_t s);
 
 }  // namespace anvil

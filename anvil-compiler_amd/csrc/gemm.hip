@@ -33,35 +33,12 @@
 
 namespace anvil {
 
-// One 16-byte K chunk of one operand row, zero outside [0, rows) x [0, K).
-template <bool VEC>
-__device__ __forceinline__ v4i load_chunk(const int8_t* __restrict__ base, long long ld, int row, int rows, int k,
-                                          int K) {
-  v4i v = {0, 0, 0, 0};
-  if (row >= rows) return v;
-  const int8_t* p = base + (long long)row * ld + k;
-  if (VEC) {
-    if (k < K) v = *reinterpret_cast<const v4i*>(p);
-  } else {
-    unsigned w[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (k + i < K) w[i >> 2] |= (unsigned)(uint8_t)p[i] << (8 * (i & 3));
-    v = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-  }
-  return v;
-}
-
-template <bool CHECKED>
-__device__ __forceinline__ int rq(int acc, const GemmArgs& g, int lo, int hi, unsigned& bad) {
-  if (CHECKED) return requant_checked(acc, g.mult, g.shift, (long long)g.rnd, lo, hi, bad);
-  const int v = (acc * g.mult + g.rnd) >> g.shift;     // the static proof keeps acc * M + rnd inside int32
-  return min(max(v, lo), hi);
-}
-
-template <int BM, int BN, int BK, int WGM, int PF, int OSZ, bool CHECKED, bool VEC>
-__global__ __launch_bounds__(G_THREADS) void gemm_i8_kernel(GemmArgs g) {
-  constexpr int WGN = 4 / WGM;                           // waves along M x along N
+// Unproven graphs (64-bit requant checked against int32), operands at any alignment: 16 bytes a load there too (1000 x 1001
+// x 1003: 20 us, byte by byte 103), and without row_chunk's shifts where a whole stage is inside the rows (4096 x 3072 x
+// 3072: 99 us, 231 with them).
+template <int BM, int BN, int BK, int OSZ>
+__global__ __launch_bounds__(G_THREADS) void gemm_i8_checked(GemmArgs g) {
+  constexpr int WGM = 2, WGN = 2;                        // waves along M x along N
   constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
   static_assert(WGM * WGN == 4 && TM >= 1 && TN >= 1, "wave grid");
   constexpr int CPR = BK / 16;
@@ -100,27 +77,40 @@ __global__ __launch_bounds__(G_THREADS) void gemm_i8_kernel(GemmArgs g) {
 
   const int lc = t % CPR, lr = t / CPR;
   constexpr int RSTEP = G_THREADS / CPR;
-  // PF register sets of staged global loads: the loads of stage s are issued PF iterations before stage s is
-  // written to LDS, so PF iterations of MFMA work cover their latency.
-  v4i ra[PF][A_PASS], rb[PF][B_PASS];
-  auto gload = [&](int set, int k0) {
+  v4i ra[A_PASS], rb[B_PASS];                            // the next stage, loaded while this one feeds the MFMAs
+  auto gload = [&](int k0) {
+    auto load = [&](auto whole_c) {
+      constexpr bool WHOLE = decltype(whole_c)::value;   // every K byte of the stage is inside the rows
+      auto chunk = [&](const int8_t* base, long long ld, int r, int rows) {
+        v4i v = {0, 0, 0, 0};
+        if (r >= rows) return v;
+        const int8_t* row = base + r * ld;
+        if (!WHOLE) return row_chunk(row, k0 + lc * 16, K);
+        __builtin_memcpy(&v, row + k0 + lc * 16, 16);
+        return v;
+      };
 #pragma unroll
-    for (int p = 0; p < A_PASS; ++p) ra[set][p] = load_chunk<VEC>(A, g.lda, lr + RSTEP * p, rows_a, k0 + lc * 16, K);
+      for (int p = 0; p < A_PASS; ++p) ra[p] = chunk(A, g.lda, lr + RSTEP * p, rows_a);
 #pragma unroll
-    for (int p = 0; p < B_PASS; ++p) rb[set][p] = load_chunk<VEC>(B, g.ldb, lr + RSTEP * p, rows_b, k0 + lc * 16, K);
+      for (int p = 0; p < B_PASS; ++p) rb[p] = chunk(B, g.ldb, lr + RSTEP * p, rows_b);
+    };
+    if (k0 + BK <= K)
+      load(std::true_type{});
+    else
+      load(std::false_type{});
   };
-  auto lstore = [&](int set, int buf) {
+  auto lstore = [&](int buf) {
     int8_t* As = smem + buf * STAGE;
     int8_t* Bs = As + BM * BK;
 #pragma unroll
     for (int p = 0; p < A_PASS; ++p) {
       const int r = lr + RSTEP * p;
-      *reinterpret_cast<v4i*>(As + r * BK + swz<BK>(r, lc) * 16) = ra[set][p];
+      *reinterpret_cast<v4i*>(As + r * BK + swz<BK>(r, lc) * 16) = ra[p];
     }
 #pragma unroll
     for (int p = 0; p < B_PASS; ++p) {
       const int r = lr + RSTEP * p;
-      *reinterpret_cast<v4i*>(Bs + r * BK + swz<BK>(r, lc) * 16) = rb[set][p];
+      *reinterpret_cast<v4i*>(Bs + r * BK + swz<BK>(r, lc) * 16) = rb[p];
     }
   };
 
@@ -156,22 +146,14 @@ __global__ __launch_bounds__(G_THREADS) void gemm_i8_kernel(GemmArgs g) {
   };
 
   const int nk = (K + BK - 1) / BK;
-#pragma unroll
-  for (int s = 0; s < PF; ++s)
-    if (s < nk) gload(s, s * BK);
-  lstore(0, 0);
+  gload(0);
+  lstore(0);
   __syncthreads();
-  for (int kt0 = 0; kt0 < nk; kt0 += PF) {
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      const int kt = kt0 + u;
-      if (kt < nk) {
-        if (kt + PF < nk) gload(u, (kt + PF) * BK);          // stage kt + PF has the parity of stage kt
-        compute(kt & 1);
-        if (kt + 1 < nk) lstore((u + 1) % PF, (kt + 1) & 1);
-        __syncthreads();
-      }
-    }
+  for (int kt = 0; kt < nk; ++kt) {
+    if (kt + 1 < nk) gload((kt + 1) * BK);
+    compute(kt & 1);
+    if (kt + 1 < nk) lstore((kt + 1) & 1);
+    __syncthreads();
   }
 
   // epilogue: requant (+ LUT) into an LDS row-major staging tile, then 16-byte global stores
@@ -188,7 +170,7 @@ __global__ __launch_bounds__(G_THREADS) void gemm_i8_kernel(GemmArgs g) {
         int v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          v[e] = rq<CHECKED>(acc[i][j][4 * q + e], g, lo, hi, bad);
+          v[e] = requant_checked(acc[i][j][4 * q + e], g.mult, g.shift, (long long)g.rnd, lo, hi, bad);
           if (OSZ == 1 && g.lut) v[e] = lut_s[(uint8_t)v[e]];
         }
         int8_t* dst = smem + m_l * SROW + n_l * OSZ;
@@ -200,7 +182,7 @@ __global__ __launch_bounds__(G_THREADS) void gemm_i8_kernel(GemmArgs g) {
           *reinterpret_cast<unsigned*>(dst + 4) = (unsigned)(v[2] & 0xffff) | ((unsigned)v[3] << 16);
         }
       }
-  if (CHECKED && bad) raise_flag(g.flags, FLAG_OVERFLOW);
+  if (bad) raise_flag(g.flags, FLAG_OVERFLOW);
   __syncthreads();
 
   constexpr int CH_ROW = BN * OSZ / 16;                  // 16-byte chunks per staged row
@@ -1380,34 +1362,14 @@ static void launch_fast_choice(GemmArgs& g, int osz, int batch, hipStream_t s, i
   }
 }
 
-template <int BM, int BN, int BK, int WGM, int PF, bool CHECKED>
-static void launch_cfg(GemmArgs& g, int osz, bool vec, int batch, hipStream_t s) {
-  g.tiles_m = (g.M + BM - 1) / BM;
-  g.tiles_n = (g.N + BN - 1) / BN;
-  dim3 grid(g.tiles_m * g.tiles_n, batch);
-  if (osz == 1) {
-    if (vec)
-      ANVIL_LAUNCH((gemm_i8_kernel<BM, BN, BK, WGM, PF, 1, CHECKED, true>), grid, dim3(G_THREADS), 0, s, g);
-    else
-      ANVIL_LAUNCH((gemm_i8_kernel<BM, BN, BK, WGM, PF, 1, CHECKED, false>), grid, dim3(G_THREADS), 0, s, g);
-  } else {
-    if (vec)
-      ANVIL_LAUNCH((gemm_i8_kernel<BM, BN, BK, WGM, PF, 2, CHECKED, true>), grid, dim3(G_THREADS), 0, s, g);
-    else
-      ANVIL_LAUNCH((gemm_i8_kernel<BM, BN, BK, WGM, PF, 2, CHECKED, false>), grid, dim3(G_THREADS), 0, s, g);
-  }
-}
-
-// Tile shape by problem: 128 x 128 for checked runs (its epilogue keeps the 64-bit checks in registers) and small
-// problems, 256 x 64 with the four waves stacked along M when N <= 64 (attention's P.V), 256 x 256 otherwise.
-static void launch_gemm(GemmArgs& g, bool checked, int osz, bool vec, int batch, hipStream_t s) {
-  if (checked) return launch_cfg<128, 128, 64, 2, 1, true>(g, osz, vec, batch, s);
-  if (g.N <= 64)
-    launch_cfg<256, 64, 64, 4, 2, false>(g, osz, vec, batch, s);
-  else if (g.M <= 128 || g.N <= 128)
-    launch_cfg<128, 128, 64, 2, 2, false>(g, osz, vec, batch, s);
+static void launch_checked(GemmArgs& g, int osz, int batch, hipStream_t s) {
+  g.tiles_m = (g.M + 127) / 128;
+  g.tiles_n = (g.N + 127) / 128;
+  const dim3 grid(g.tiles_m * g.tiles_n, batch);
+  if (osz == 1)
+    ANVIL_LAUNCH((gemm_i8_checked<128, 128, 64, 1>), grid, dim3(G_THREADS), 0, s, g);
   else
-    launch_cfg<256, 256, 64, 2, 2, false>(g, osz, vec, batch, s);
+    ANVIL_LAUNCH((gemm_i8_checked<128, 128, 64, 2>), grid, dim3(G_THREADS), 0, s, g);
 }
 
 // Static split-K scratch of anvil_gemm_i8_noalloc: SCRATCH_SUMS int32 partial sums. Each device holds its own copy
@@ -1468,7 +1430,7 @@ struct AddEpilogue {
 struct Prepared {
   GemmArgs g;
   int osz, batch;
-  bool checked, vec, fast, mul24, force_split;
+  bool checked, fast, mul24, force_split;
 };
 
 // The deep-pipelined kernel (gemm_deep.hip, 64 x 64 tiles) takes a product, or a group, of at most two tiles a CU: the
@@ -1595,7 +1557,6 @@ static int gemm_prepare(anvil_ctx* ctx, const int8_t* A, const int8_t* Bt, void*
   p.osz = osz;
   p.batch = batch0 * batch1;
   p.checked = checked;
-  p.vec = vec;
   p.fast = fast;
   p.mul24 = (flags & ANVIL_GEMM_MUL24) != 0;
   p.force_split = (flags & ANVIL_GEMM_SPLITK) != 0;
@@ -1623,7 +1584,10 @@ static int ensure_workspace(anvil_ctx* ctx, long long sums) {
 // first use), or with `noalloc` in the static scratch, within whose size it must then fit.
 static int gemm_launch(anvil_ctx* ctx, Prepared& p, bool noalloc = false) {
   if (!p.fast) {
-    launch_gemm(p.g, p.checked, p.osz, p.vec, p.batch, ctx->stream);
+    if (p.checked)
+      launch_checked(p.g, p.osz, p.batch, ctx->stream);
+    else
+      launch_any(p.g, p.osz, p.mul24, p.batch, ctx->num_cu, ctx->stream);
     return ANVIL_OK;
   }
   int splits = 0, kchunk = 0;
