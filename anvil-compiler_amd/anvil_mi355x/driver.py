@@ -95,6 +95,9 @@ def _checked_graph(module, consts, prove=True):
 
 
 PINNED_MAX = 1 << 28       # read-back buffers up to this size download into page-locked host memory
+# run()'s float inputs and token ids up to this size are read by their kernel where the host wrote them: with the wait
+# 17 us against 35 for 8 KiB through a device copy, 48 against 61 at 1 MiB, no difference at 4 MiB
+ZERO_COPY_MAX = 1 << 20
 PINNED_PLAN_MAX = 1 << 30  # page-locked read-back memory one plan keeps at most; larger reads go pageable
 
 
@@ -110,6 +113,8 @@ class _Plan:
         self.norm_of: dict = {}        # fused add_requant -> the rmsnorm_int of its sum that may share its epilogue
         self.fused_norms: set = set()  # rmsnorm_int ops computed in a GEMM epilogue
         self.stage: dict = {}          # device staging buffers of float inputs and token ids
+        self.host_in: dict = {}        # page-locked inputs of run(), by sym
+        self.reads: dict = {}          # read()'s buffers by its syms
         self.host_stage: dict = {}     # page-locked host buffers the read-back downloads into, by device buffer
         self.graph = None              # the steps captured as one HIP graph (run(..., graph=True))
         self.launched = False          # an eager launch has run
@@ -184,6 +189,8 @@ class CompiledModel:
         self._const_bt_host = {}
         self._plans = {}
         self._row_streams = {}
+        self._by_sym = {op.sym_str: op.result for op in self.ops if op.sym_str is not None}
+        self._const_syms = frozenset(op.sym_str for op in self.ops if isinstance(op, g.ConstOp))
         self.row_programs = True          # runs of row-wise ops as one anvil_row_program launch (rowprog.py)
         self.group_gemms = True           # independent consecutive GEMMs as one anvil_gemm_i8_group call
 
@@ -1005,8 +1012,28 @@ class CompiledModel:
             raise ValueError(f"keep must be 'outputs' or 'all', not {keep!r}")
         return [s for s in dict.fromkeys(syms) if s is not None]
 
-    def upload_inputs(self, plan, ints: dict):
-        """Integer inputs, or float inputs (quantized on the device), into the plan's input buffers."""
+    def _host_input(self, plan, sym, a):
+        """The address of a copy of `a` in page-locked memory of the plan, for kernels to read in place, or None (large
+        inputs, a stand-in device). The caller waits for those kernels before the next input of this plan."""
+        if a.nbytes > ZERO_COPY_MAX or not hasattr(self.dev, "fetch"):
+            return None
+        h = plan.host_in.get(sym)
+        if h is None or h.nbytes < a.nbytes:
+            h = plan.host_in[sym] = self.dev.host_alloc(a.nbytes)
+        h.array(a.dtype, a.size)[:] = a.reshape(-1)
+        return h.ptr
+
+    def upload_inputs(self, plan, ints: dict, deferred=False) -> bool:
+        """Integer inputs, or float inputs (quantized on the device), into the plan's input buffers. deferred: the only
+        input, floats of up to ZERO_COPY_MAX bytes, is quantized from page-locked memory without a wait and True
+        returned: the caller's next check reports its NaN or infinite values, and waits for the kernel."""
+        if deferred and len(self.input_ops) == 1:
+            op = self.input_ops[0]
+            x, v = ints[op.sym_str], plan.views[op.result]
+            at = self._host_input(plan, op.sym_str, x.a) if isinstance(x, _FloatInput) else None
+            if at is not None:
+                self.dev.quantize(at, x.a.dtype == np.float64, self.scale(op.sym_str), x.a.size, v.ptr, v.dtype)
+                return True
         for op in self.input_ops:
             v = plan.views[op.result]
             x = ints[op.sym_str]
@@ -1023,9 +1050,11 @@ class CompiledModel:
                     raise
             else:
                 v.buf.mem.upload(np.ascontiguousarray(x).astype(rt.NP_DTYPE[v.dtype]))
+        return False
 
-    def upload_tokens(self, plan, ids):
-        """Token ids through the embedding prelude into the input buffer: gather, add and quantize on the device."""
+    def upload_tokens(self, plan, ids, deferred=False):
+        """Token ids through the embedding prelude into the input buffer: gather, add and quantize on the device.
+        deferred: the ids are read from page-locked memory, until the caller's next wait."""
         if self._embed_dev is None:
             wte, wpe = self.embedding
             self._embed_dev = (self.dev.upload(wte), self.dev.upload(wpe), wte.shape[0])
@@ -1033,8 +1062,11 @@ class CompiledModel:
         sym = self.inputs[0]
         v = plan.views[self.input_ops[0].result]
         T, Cdim = self.meta[sym][1]
-        stage = self._stage(plan, sym + ".ids", ids.nbytes)
-        stage.upload(np.ascontiguousarray(ids, dtype=np.int64))
+        ids = np.ascontiguousarray(ids, dtype=np.int64)
+        stage = self._host_input(plan, sym, ids) if deferred else None
+        if stage is None:
+            stage = self._stage(plan, sym + ".ids", ids.nbytes)
+            stage.upload(ids)
         self.dev.embed_quantize(stage, ids.size, T, Cdim, wte_d, vocab, wpe_d, self.scale(sym), v.ptr, v.dtype)
 
     def _stage(self, plan, key, nbytes):
@@ -1073,35 +1105,61 @@ class CompiledModel:
             times[label] = times.get(label, 0.0) + 1e3 * self.dev.elapsed_ms(4, 5)
         return times
 
-    def read(self, plan, syms, nb=None, batch=True, narrow=None) -> dict:
-        """sym -> int64 array of each of syms, read back from the device. A device buffer of up to PINNED_MAX bytes
-        is downloaded into a page-locked buffer of the plan (DMA straight into it, no pageable staging) and widened
-        from there, while the plan's page-locked buffers stay within PINNED_PLAN_MAX bytes in total; beyond that a
+    def _read_buffers(self, plan, syms):
+        """The device buffers that hold syms, as (the fetch of those with a page-locked buffer in the plan, or None,
+        those buffers by id, the others by id)."""
+        pinned, plain = {}, {}
+        for s in syms:
+            v = plan.views[self._by_sym[s]]
+            key = id(v.buf)
+            if key in pinned or key in plain:
+                continue
+            into = None
+            if v.buf.nbytes <= PINNED_MAX:
+                into = plan.host_stage.get(key)
+                if into is None or into.nbytes < v.buf.nbytes:
+                    held = sum(h.nbytes for k, h in plan.host_stage.items() if k != key)
+                    into = None
+                    if held + v.buf.nbytes <= PINNED_PLAN_MAX:
+                        into = plan.host_stage[key] = self.dev.host_alloc(v.buf.nbytes)
+            if into is None:
+                plain[key] = v
+            else:
+                pinned[key] = (v, into)
+        fetch = None
+        if hasattr(self.dev, "fetch"):
+            fetch = self.dev.fetch([(v.buf.mem, h, v.buf.nbytes) for v, h in pinned.values()])
+        return fetch, pinned, plain
+
+    def read(self, plan, syms, nb=None, batch=True, narrow=None, check=False) -> dict:
+        """sym -> int64 array of each of syms, read back from the device; check: as the device's sync() reports
+        violations, first. Device buffers of up to PINNED_MAX bytes are copied into page-locked buffers of the plan, with
+        one wait for all of them (Device.fetch), and widened from there, while the plan's page-locked buffers stay within PINNED_PLAN_MAX bytes in total; beyond that a
         read downloads into ordinary (pageable) memory. With a dict `narrow`, also sym -> the same values as a view at their stored dtype (no copy, into
         that buffer: use it before the plan's next read). Reads of one plan from several threads need the device
         lock around them, as run() holds it."""
-        by_sym = {op.sym_str: op.result for op in self.ops if op.sym_str is not None}
+        got = plan.reads.get(tuple(syms))
+        if got is None:
+            got = plan.reads[tuple(syms)] = self._read_buffers(plan, syms)
+        fetch, pinned, plain = got
+        if fetch is not None:
+            fetch(check)
+        elif check:
+            self.dev.sync()
         cache, out = {}, {}
+        for key, (v, h) in pinned.items():
+            n, dt = v.buf.nbytes // v.itemsize, rt.NP_DTYPE[v.dtype]
+            cache[key] = h.array(dt, n) if fetch is not None else v.buf.mem.download((n,), dt, into=h)
+        for key, v in plain.items():
+            cache[key] = v.buf.mem.download((v.buf.nbytes // v.itemsize,), rt.NP_DTYPE[v.dtype])
         for s in syms:
-            v = plan.views[by_sym[s]]
-            key = id(v.buf)
-            if key not in cache:
-                into = None
-                if v.buf.nbytes <= PINNED_MAX:
-                    into = plan.host_stage.get(key)
-                    if into is None or into.nbytes < v.buf.nbytes:
-                        held = sum(h.nbytes for k, h in plan.host_stage.items() if k != key)
-                        if held + v.buf.nbytes <= PINNED_PLAN_MAX:
-                            into = plan.host_stage[key] = self.dev.host_alloc(v.buf.nbytes)
-                        else:
-                            into = None
-                cache[key] = v.buf.mem.download((v.buf.nbytes // v.itemsize,), rt.NP_DTYPE[v.dtype], into=into)
-            whole = batch or by_sym[s] in self.is_const
-            a = v.read(cache[key])
+            v = plan.views[self._by_sym[s]]
+            base = v.view(cache[id(v.buf)])
+            whole = batch or self._by_sym[s] in self.is_const
+            a = hostpar.astype(base, np.int64)
             out[s] = a if whole else a[0]
             if narrow is not None:
-                n = v.view(cache[key])
-                narrow[s] = n if whole else n[0]
+                narrow[s] = base if whole else base[0]
         return out
 
     AUTO_EAGER_RUNS = 2                # eager runs a plan times before its graph is captured and timed
@@ -1144,30 +1202,36 @@ class CompiledModel:
             ints_in, nb = self._bind_inputs(x, quantized, batch)
         plan = self.plan(nb, keep)
         with self.dev.lock:
-            if tokens:
-                self.upload_tokens(plan, ids)
-            else:
-                self.upload_inputs(plan, ints_in)
-            auto = graph is None and not profile
-            if auto:
-                graph = self._auto_graph(plan)
-            captured = bool(graph) and plan.graph is None
-            self.dev.record(2)
-            times = self.launch(plan, profile, graph)
-            self.dev.record(3)
-            self.dev.sync()
+            floats = False
+            narrow = {}
+            try:
+                if tokens:
+                    self.upload_tokens(plan, ids, deferred=True)
+                else:
+                    floats = self.upload_inputs(plan, ints_in, deferred=not profile)
+                auto = graph is None and not profile
+                if auto:
+                    graph = self._auto_graph(plan)
+                captured = bool(graph) and plan.graph is None
+                self.dev.record(2)
+                times = self.launch(plan, profile, graph)
+                self.dev.record(3)
+                ints = self.read(plan, syms, nb, batch, narrow, check=True)
+            except BaseException as e:
+                if hasattr(self.dev, "fetch"):
+                    self.dev.fetch([])()              # nothing reads this run's host input any more
+                if floats and isinstance(e, ValueError) and "NaN or infinite" in str(e):
+                    raise ValueError(f"input {self.inputs[0]!r} has NaN or infinite values") from None
+                raise
             total_ms = self.dev.elapsed_ms(2, 3)
             if auto:
                 self._note_auto(plan, graph, captured, total_ms)
-            narrow = {}
-            ints = self.read(plan, syms, nb, batch, narrow)
             # from the stored dtype (1-2 bytes an element), before another run reuses the plan's host buffers
             outs = [self.dequantize(s, narrow[s]) for s in self.outputs]
         cycles = {label: (times.get(label) if profile else None) for label, _, _ in plan.steps}
-        consts = frozenset(op.sym_str for op in self.ops if isinstance(op, g.ConstOp))
         result = {"device_ms": total_ms, "batch": nb, "kernels": len(plan.steps), "footprint": plan.footprint,
                   "hip_graph": bool(graph) and not profile}
-        return RunOutput(outs[0], outs, ints, cycles, result, None, consts, self)
+        return RunOutput(outs[0], outs, ints, cycles, result, None, self._const_syms, self)
 
     def summary(self) -> str:
         plan = self.plan(1)

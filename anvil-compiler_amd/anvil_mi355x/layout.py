@@ -11,7 +11,6 @@ from dataclasses import dataclass
 
 import numpy as np
 
-from . import hostpar
 
 ITEMSIZE = {"i8": 1, "i16": 2, "i32": 4}
 
@@ -112,10 +111,6 @@ class View:
             return blocks.reshape(self.dims)
         return np.lib.stride_tricks.as_strided(base[self.offset:], shape=self.dims,
                                                strides=tuple(s * isz for s in self.strides))
-
-    def read(self, base: np.ndarray) -> np.ndarray:
-        """This view of `base` as a new int64 array."""
-        return hostpar.astype(self.view(base), np.int64)
 
 
 def nocopy_strides(dims, strides, newdims):

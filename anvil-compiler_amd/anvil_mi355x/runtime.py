@@ -49,6 +49,7 @@ SIGNATURES = {
     "anvil_host_free": [_p, _p],
     "anvil_upload": [_p, _p, _p, _sz],
     "anvil_download": [_p, _p, _p, _sz],
+    "anvil_fetch": [_p, _i, _p, _p, _p, _i],
     "anvil_zero": [_p, _p, _sz],
     "anvil_graph_begin": [_p],
     "anvil_graph_end": [_p, C.POINTER(_p)],
@@ -243,6 +244,18 @@ class HipGraph:
             pass
 
 
+class Fetch:
+    """anvil_fetch of a list of buffers, which it keeps alive."""
+
+    def __init__(self, dev: "Device", items):
+        self.dev, self.items, n = dev, list(items), len(items)
+        self.args = (n, (C.c_void_p * max(1, n))(*[b.ptr for b, _, _ in items]),
+                     (C.c_void_p * max(1, n))(*[h.ptr for _, h, _ in items]), (_sz * max(1, n))(*[k for _, _, k in items]))
+
+    def __call__(self, check=False):
+        self.dev.lib.call("anvil_fetch", self.dev.ctx, *self.args, int(check))
+
+
 class RowProgram:
     """A row program of a Device (anvil_row_create), run by launch(); freed when collected."""
 
@@ -320,6 +333,11 @@ class Device:
 
     def sync(self):
         self.lib.call("anvil_sync", self.ctx)
+
+    def fetch(self, items) -> "Fetch":
+        """Copies of device buffers into page-locked ones, [(DeviceBuffer, HostBuffer, bytes)], as a callable: one wait
+        for all of them, and with check=True what sync() reports."""
+        return Fetch(self, items)
 
     def zero(self, ptr, nbytes: int):
         self.lib.call("anvil_zero", self.ctx, C.c_void_p(_ptr(ptr)), C.c_size_t(nbytes))

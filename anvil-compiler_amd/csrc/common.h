@@ -38,6 +38,7 @@ struct anvil_ctx {
   int* ws = nullptr;
   long long ws_elems = 0;
   std::vector<int*> ws_retired;
+  unsigned* host_flags = nullptr; // page-locked word the flags are fetched into
 };
 
 namespace anvil {

@@ -59,6 +59,10 @@ int anvil_host_free(anvil_ctx* ctx, void* hptr);
 /* Host <-> device copies on the context's stream; they complete before the call returns. */
 int anvil_upload(anvil_ctx* ctx, void* dst, const void* src, size_t bytes);
 int anvil_download(anvil_ctx* ctx, void* dst, const void* src, size_t bytes);
+/* Copy n device buffers (16-byte aligned) into page-locked host memory (anvil_host_alloc), in stream order, and wait for
+ * the stream: one wait for all of them. check != 0: also report (and clear) device-side contract violations as
+ * anvil_sync does, a non-finite float input before any other; the copies then hold unspecified values. */
+int anvil_fetch(anvil_ctx* ctx, int n, const void* const* src, void* const* dst, const size_t* bytes, int check);
 /* Zero `bytes` of device memory with a fill kernel (safe inside a captured graph). */
 int anvil_zero(anvil_ctx* ctx, void* dst, size_t bytes);
 
