@@ -1296,11 +1296,11 @@ static void launch_splitk(GemmArgs& g, int osz, hipStream_t s) {
   }
 }
 
-// Whether a fast-path product splits K, and into how many chunks: a single product (batch 1, no causal mode or fused
-// add) with K >= 2048 whose 128 x 128 output tiles fill at most a quarter of the CUs splits into two to SPLITK_MAX
-// chunks of whole 64-byte K blocks; `force` (ANVIL_GEMM_SPLITK) splits any such product. Measured on MI355X (two
-// launches, partial tiles through the workspace): 256 x 3072 x 3072 (48 tiles) 22.1 -> 17.8 us; at K = 768
-// (256 x 768 x 768, 12 tiles) the second launch costs more than the split saves, 11.4 -> 13.3 us.
+// Whether a fast-path product splits K, and into how many chunks: `force` (ANVIL_GEMM_SPLITK) splits any single product
+// (batch 1, no causal mode or fused add) into two to SPLITK_MAX chunks of whole 64-byte K blocks. Without it the rule is
+// K >= 2048 with 128 x 128 output tiles on at most a quarter of the CUs; gemm_i8_deep serves those first (256 x 3072 x
+// 3072: 8.7 us, 17.8 split), so it decides only under a pinned tile shape and that a group's members run one by one.
+// Two launches, partial tiles through the workspace; the one-pass 128 x 128 kernel took 22.1 us there.
 static bool splitk_plan(const GemmArgs& g, int batch, int num_cu, bool force, int& splits, int& kchunk) {
   if (batch != 1 || g.causal != 0 || g.res) return false;
   const long long tiles = (long long)((g.M + 127) / 128) * ((g.N + 127) / 128);

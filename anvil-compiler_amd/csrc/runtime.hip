@@ -3,6 +3,7 @@
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <utility>
 #include <vector>
 
@@ -29,6 +30,7 @@ struct LaunchRecord {
 struct LaunchList {
   std::vector<LaunchRecord> launches;
   hipGraphExec_t exec = nullptr;
+  bool incomplete = false;             // a launch could not be noted
 };
 
 // the lists this thread is recording, innermost last, each with the stream it records
@@ -38,12 +40,17 @@ struct Recording {
 };
 static thread_local std::vector<Recording> g_recordings;
 
-static hipError_t note_launch(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
-                              const unsigned short* sizes, int n) {
+// A launch that cannot be noted has still run: it only spoils the recordings, which then end in an error.
+static void note_launch(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
+                        const unsigned short* sizes, int n) try {
   for (Recording& rec : g_recordings) {
     if (rec.stream != s) continue;
     LaunchRecord r{sym, nullptr, grid, block, lds, {}, {}, {sizes, sizes + n}};
-    if (hipError_t e = hipGetFuncBySymbol(&r.fn, sym); e != hipSuccess) return e;
+    if (hipGetFuncBySymbol(&r.fn, sym) != hipSuccess) {
+      (void)hipGetLastError();
+      rec.list->incomplete = true;
+      continue;
+    }
     size_t total = 0;
     for (int i = 0; i < n; ++i) total = (total + 15) / 16 * 16 + sizes[i];
     r.bytes.resize(total + 1);
@@ -56,7 +63,9 @@ static hipError_t note_launch(const void* sym, dim3 grid, dim3 block, unsigned l
     }
     rec.list->launches.push_back(std::move(r));   // moving the vectors keeps their storage, and so the pointers
   }
-  return hipSuccess;
+} catch (const std::bad_alloc&) {
+  for (Recording& rec : g_recordings)
+    if (rec.stream == s) rec.list->incomplete = true;
 }
 
 int launch_kernel(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
@@ -69,7 +78,7 @@ int launch_kernel(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStrea
   } else {
     e = hipLaunchKernel(sym, grid, block, args, lds, s);
   }
-  if (e == hipSuccess && !g_recordings.empty()) e = note_launch(sym, grid, block, lds, s, args, sizes, n);
+  if (e == hipSuccess && !g_recordings.empty()) note_launch(sym, grid, block, lds, s, args, sizes, n);
   return e == hipSuccess ? ANVIL_OK : hip_fail(e, "kernel launch");
 }
 
@@ -350,7 +359,7 @@ int anvil_graph_end(anvil_ctx* ctx, void** graph) {
   size_t nodes = 0;
   e = hipGraphGetNodes(g, nullptr, &nodes);
   if (!l) l = new LaunchList();
-  if (e != hipSuccess || nodes != l->launches.size()) {
+  if (e != hipSuccess || nodes != l->launches.size() || l->incomplete) {
     l->launches.clear();
     e = hipGraphInstantiate(&l->exec, g, nullptr, nullptr, 0);
   }
@@ -376,8 +385,14 @@ int anvil_record_end(anvil_ctx* ctx, void** list) {
     delete l;
     return set_error(ANVIL_E_VALUE, "anvil_record_end: null output pointer");
   }
+  *list = nullptr;
+  if (!l) return set_error(ANVIL_E_VALUE, "anvil_record_end: nothing is being recorded on this thread");
+  if (l->incomplete) {
+    delete l;
+    return set_error(ANVIL_E_RUNTIME, "anvil_record_end: a launch could not be recorded");
+  }
   *list = l;
-  return l ? ANVIL_OK : set_error(ANVIL_E_VALUE, "anvil_record_end: nothing is being recorded on this thread");
+  return ANVIL_OK;
 }
 
 int anvil_graph_launch(anvil_ctx* ctx, void* graph) {
