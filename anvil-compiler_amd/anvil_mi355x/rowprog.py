@@ -101,38 +101,37 @@ def _row_operands(op) -> list:
 
 
 def find(cm, nb) -> list:
-    """The graph's runs of at least two row-wise ops, a product among them. Views (transposes, reshapes) between them cost no launch: a run
-    goes on past a view of one of its values until an op reads that view."""
+    """The graph's runs of at least two row-wise ops, a product among them. A run is planned where its first op stands, so
+    its ops may read only what is planned by then: each other's results, and values from before it. Graph inputs and views
+    (transposes, reshapes) inside a run cost no launch: it goes on past them until an op reads one."""
     if not cm.proven:
         return []
     progs, cur, T = [], [], None
-    inside, viewed = set(), set()       # values computed in the open run, and views of them
+    late = set()                        # inputs and views that stand inside the open run
 
     def close():
         nonlocal cur
         if len(cur) > 1 and any(isinstance(op, (g.QLinearOp, g.QMatmulOp)) for op in cur):
             progs.append(Program(cur))
         cur = []
-        inside.clear()
-        viewed.clear()
+        late.clear()
 
     for op in cm.ops:
-        if isinstance(op, (g.InputOp, g.ConstOp)):
+        if isinstance(op, g.ConstOp):
             continue
         r = op.results[0]
-        if isinstance(op, (g.TransposeOp, g.ReshapeOp)):
-            if op.x in inside or op.x in viewed:
-                viewed.add(r)
+        if isinstance(op, (g.InputOp, g.TransposeOp, g.ReshapeOp)):
+            if cur:
+                late.add(r)
             continue
         if not _eligible(cm, op, nb):
             close()
             continue
         rows = g.qt(r).dims[0]
-        if (cur and rows != T) or any(v in viewed for v in _row_operands(op)):
+        if (cur and rows != T) or any(v in late for v in _row_operands(op)):
             close()
         T = rows
         cur.append(op)
-        inside.add(r)
     close()
     return progs
 

@@ -12,6 +12,7 @@ import fake_device
 import helpers
 from anvil_mi355x import models, rowprog
 from anvil_mi355x import runtime as rt
+from anvil_mi355x.ir import GraphBuilder
 from oracle import interp
 from oracle import semantics as sem
 
@@ -153,6 +154,41 @@ def test_planner_runs_the_frozen_models_as_row_programs(monkeypatch, model, keep
     lim = 128 if model == "v1" else 1 << 15
     check(module, consts, (module, consts), np.random.default_rng(3).integers(-lim, lim, (3, 16, 32)), keep, True)
     assert [c[0] for c in dev.calls].count("row_program") == 3 and len(dev.calls) == 5
+
+
+def late_graph(late):
+    """h = x w, then r = h + z, where z is an input after h, or a view made after h of an earlier input."""
+    rng = np.random.default_rng(21)
+    bld = GraphBuilder("late")
+    x = bld.input("x", [16, 32])
+    z = bld.input("z", {"reshape": [16, 2, 16], "transpose": [32, 16]}[late]) if late != "input" else None
+    weight = lambda s: bld.const(s, [32, 32], value=rng.integers(-128, 128, (32, 32)))     # noqa: E731
+    h = bld.qlinear("h", x, weight("w"), 3, 13)
+    h2 = bld.qlinear("h2", h, weight("w2"), 3, 13)
+    if late == "input":
+        zr = bld.input("z", [16, 32])
+    else:
+        zr = bld.reshape("zr", z, [16, 32]) if late == "reshape" else bld.transpose("zr", z, [1, 0])
+    r = bld.add_requant("r", h2, zr, 100, 90, 8)
+    bld.output(bld.qlinear("y", r, weight("w3"), 3, 13))
+    return bld.module()
+
+
+@pytest.mark.parametrize("late", ["input", "reshape", "transpose"])
+@pytest.mark.parametrize("keep", ["outputs", "all"])
+def test_a_run_ends_before_an_operand_that_stands_inside_it(monkeypatch, late, keep):
+    dev = RowFake()
+    monkeypatch.setattr(rt, "device", lambda index=0: dev)
+    m = late_graph(late)
+    cm = anvil_mi355x.compile(m)
+    rng = np.random.default_rng(5)
+    x = {s: rng.integers(-128, 128, (3, *cm.meta[s][1])) for s in cm.inputs}
+    res = cm.run([x[s] for s in cm.inputs], "mi355x", batch=True, keep=keep, quantized=True)
+    want = interp.run(m, x, {}, batch=True, fast=True)
+    for k in res.ints:
+        assert np.array_equal(res.ints[k], want.values[k]), k
+    # rows of the transposed input are no rows of one stride: those ops run one by one
+    assert [c[0] for c in dev.calls].count("row_program") == (1 if late == "transpose" else 2)
 
 
 @pytest.mark.gpu
