@@ -220,8 +220,8 @@ class CompiledModel:
 
     def _chain_of(self, o_op):
         """(scores matmul, softmax) when o_op is the P.V product of a chain the fused attention evaluates (the
-        structure only: proven, int8 throughout, scores and p read by nothing else, square scores with T up to 1024
-        and a head dim of 16, 32, 64 or 128), else None."""
+        structure only: proven, int8 throughout, q, k and v computed and of one rank, scores and p read by nothing else,
+        square scores with T up to 1024 and a head dim of 16, 32, 64 or 128), else None."""
         if not self.proven or not isinstance(o_op, g.QMatmulOp) or o_op.lut is not None:
             return None
         if g.qt(o_op.result).dtype != "i8":
@@ -236,6 +236,8 @@ class CompiledModel:
         if any(v in self.is_const or self.users.get(v, []) != [u] for v, u in ((s_op.result, sm), (sm.result, o_op))):
             return None
         sd, od = g.qt(s_op.result).dims, g.qt(o_op.result).dims
+        if any(v in self.is_const or len(g.qt(v).dims) != len(sd) for v in (s_op.a, s_op.b, o_op.b)):
+            return None                       # a const has no batch dim, a (K, N) right operand none of the heads'
         T, D = sd[-1], g.qt(s_op.a).dims[-1]
         if sd[-2] != T or T > 1024 or D not in (16, 32, 64, 128) or od[-1] != D or od[-2] != T:
             return None

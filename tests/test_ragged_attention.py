@@ -5,8 +5,10 @@ import pytest
 
 import anvil_mi355x
 import fake_device
+import test_row_program
 from anvil_mi355x import models
 from anvil_mi355x import runtime as rt
+from anvil_mi355x.ir import GraphBuilder
 from oracle import interp
 from oracle import semantics as sem
 
@@ -84,3 +86,42 @@ def test_ragged_block_matches_the_oracle(T, C, H, keep):
     want = interp.run(built.module, {"x": cm.quantize_input(x)}, built.consts, batch=True, fast=True)
     for k in res.ints:
         assert np.array_equal(res.ints[k], want.values[k]), k
+
+
+def const_operand_graph(T, const, dim=32):
+    """One head whose q, k or v is a const, over computed values otherwise."""
+    rng = np.random.default_rng([31, T])
+    bld = GraphBuilder("const_" + const)
+    x = bld.input("x", [T, dim])
+    vals = {}
+    for s in "qkv":
+        if s == const:
+            vals[s] = bld.const(s, [T, dim], value=rng.integers(-128, 128, (T, dim)))
+        else:
+            w = bld.const("w" + s, [dim, dim], value=rng.integers(-128, 128, (dim, dim)))
+            vals[s] = bld.qlinear(s, x, w, 3, 13)
+    scores = bld.qmatmul("s", vals["q"], bld.transpose("kt", vals["k"], [1, 0]), 3, 13)
+    exp = np.round(16384.0 * np.exp((np.arange(256) - 255.0) / 20))
+    p = bld.softmax_lut("p", scores, bld.const("e", [256], dtype="i32", value=exp), 127, True)
+    o = bld.qmatmul("o", p, vals["v"], 1, 7)
+    w = bld.const("wy", [dim, dim], value=rng.integers(-128, 128, (dim, dim)))
+    bld.output(bld.add_requant("r", bld.qlinear("y", o, w, 3, 13), x, 100, 90, 8))
+    return bld.module()
+
+
+@pytest.mark.parametrize("T", [5, 16, 32, 33])
+@pytest.mark.parametrize("const", ["q", "k", "v"])
+@pytest.mark.parametrize("keep", ["outputs", "all"])
+@pytest.mark.parametrize("row_programs", [False, True])
+def test_a_const_operand_leaves_the_three_ops(monkeypatch, T, const, keep, row_programs):
+    """q, k and v of a fused chain have the batch dim; a const has none."""
+    dev = test_row_program.RowFake() if row_programs else fake_device.FakeDevice()
+    monkeypatch.setattr(rt, "device", lambda index=0: dev)
+    m = const_operand_graph(T, const)
+    cm = anvil_mi355x.compile(m)
+    x = np.random.default_rng(3).integers(-128, 128, (3, T, 32))
+    res = cm.run(x, "mi355x", batch=True, keep=keep, quantized=True)
+    want = interp.run(m, {"x": x}, {}, batch=True, fast=True)
+    for k in res.ints:
+        assert np.array_equal(res.ints[k], want.values[k]), k
+    assert "softmax" in [c[0] for c in dev.calls]
