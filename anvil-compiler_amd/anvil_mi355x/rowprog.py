@@ -241,10 +241,13 @@ def _memory(view, rows, n):
     if flat is None or flat.strides[-1] != 1:
         return None
     unit = 16 // flat.itemsize
-    ld, kb = (64, flat.kb) if flat.kb else (flat.strides[0] if rows > 1 else -(-n // unit) * unit, 64)
+    if flat.kb > 64:
+        ld, kb = 64, flat.kb
+    else:                                                   # K blocks of one row (kb = 64) follow each other: row-major
+        ld, kb = (flat.strides[0] if rows > 1 else -(-n // unit) * unit), 64
     if ld % unit or kb % 16 or flat.offset % unit or (flat.kb and flat.itemsize != 1):
         return None
-    if not flat.kb and ld < n:
+    if kb == 64 and ld < n:
         return None
     return flat, ld, kb
 

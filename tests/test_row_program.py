@@ -29,7 +29,53 @@ class RowFake(fake_device.FakeDevice):
     """The stand-in with anvil_row_program, op by op on the oracle, from the C structs."""
 
     def row_program(self, *args):
+        self.check_program(*args)
         return RowFakeProgram(self, args)
+
+    @staticmethod
+    def check_program(ops, rows, seq, stream, tables, ntables):
+        """What anvil_row_create refuses."""
+        assert 1 <= len(ops) <= rowprog.OPS_MAX and 0 <= ntables <= rowprog.TABLES_MAX
+        assert rows >= 1 and seq >= 1 and rows % seq == 0 and rows < (1 << 31) - 32
+        top = norm = frags = 0
+        for i, o in enumerate(ops):
+            gemm, load = o.kind == rt.ROW_GEMM, o.kind == rt.ROW_LOAD
+            trans, only8 = gemm and o.trans, o.kind in (rt.ROW_LUT, rt.ROW_LUT_MUL)
+            chunks = -(-o.n // 32)
+            assert 16 <= o.n <= 4096 and o.n % 16 == 0 and 0 <= o.shift <= 31
+            values = [] if trans else [(o.dst, chunks, o.wide)]
+            values += [] if load else [(o.a, o.k if gemm else chunks, o.wide_a)]
+            values += [(o.b, chunks, o.wide_b)] if o.kind in (rt.ROW_ADD, rt.ROW_LUT_MUL) else []
+            for at, n, wide in values:
+                assert 0 <= at and at + n * (1 + wide) <= rowprog.SLOTS_MAX
+                top = max(top, at + n * (1 + wide))
+            assert not load or all(p.kind == rt.ROW_LOAD for p in ops[:i])
+            assert not (only8 and (o.wide or o.wide_a or o.wide_b)) and not (o.kind == rt.ROW_NORM and o.wide)
+            assert not (gemm and o.wide_a) and not (trans and o.wide)
+            if gemm:
+                assert 1 <= o.k <= rowprog.SLOTS_MAX and o.table < ntables and not (o.table >= 0 and o.wide)
+                frags += chunks * o.k
+            assert not only8 or 0 <= o.table < ntables
+            if o.m24 and o.kind == rt.ROW_ADD:
+                assert max(abs(o.mult), abs(o.mult2)) < 1 << (23 if o.wide or o.wide_a or o.wide_b else 24)
+            elif o.m24:
+                assert abs(o.mult) < 1 << 23
+            src = getattr(o, "in")
+            if load:
+                assert src and src % 16 == 0
+            if o.kind == rt.ROW_NORM:
+                assert src and src % 16 == 0 and o.lut and 1 <= o.lut_len <= rowprog.LUT_MAX and o.lut_len % 4 == 0
+                assert 0 <= o.c <= 30 and o.e >= 0
+                norm += 1024 * (-(-4 * o.lut_len // 1024) + -(-o.n // 1024))
+            if trans:
+                assert o.out and o.out % 4 == 0 and o.ld % 4 == 0 and o.kb % 4 == 0 and o.ld >= seq and o.kb >= 0
+            elif o.out or load:
+                assert (o.out or 0) % 16 == 0 and o.ld * (1 + o.wide) % 16 == 0 and o.kb % 16 == 0 and o.ld <= 1 << 24
+                blocked = not o.wide and o.kb != 64
+                assert (o.ld == 64 and o.kb >= rows * 64) if blocked else o.ld >= o.n
+        assert all(tables[i] and tables[i] % 4 == 0 for i in range(ntables))
+        assert 1024 * frags == (stream.nbytes if stream is not None else 0)
+        assert 256 * rowprog.TABLES_MAX + norm + 1024 * (frags + top) <= rowprog.LDS_MAX
 
     def run_row_program(self, ops, rows, seq, stream, tables, ntables):
         self.calls.append(("row_program", rows, seq, len(ops)))
@@ -156,6 +202,20 @@ def test_planner_runs_the_frozen_models_as_row_programs(monkeypatch, model, keep
     assert [c[0] for c in dev.calls].count("row_program") == 3 and len(dev.calls) == 5
 
 
+@pytest.mark.parametrize("C,H", [(32, 2), (32, 1), (64, 1)])
+@pytest.mark.parametrize("keep", ["outputs", "all"])
+def test_one_row_of_k_blocked_values(monkeypatch, C, H, keep):
+    """One sequence of one row: a K-blocked value's blocks follow each other, which the kernel takes as a row."""
+    dev = RowFake()
+    monkeypatch.setattr(rt, "device", lambda index=0: dev)
+    monkeypatch.setattr(rowprog, "_product_min", lambda rows: 64)
+    b = block(C, H, 1)
+    cm = check(b.module, b.consts, b, block_inputs(b, 1), keep, False)
+    assert [c[0] for c in dev.calls].count("row_program") == 2
+    if keep == "all":
+        assert any(v.kb for v in cm.plan(1, keep).views.values())
+
+
 def late_graph(late):
     """h = x w, then r = h + z, where z is an input after h, or a view made after h of an earlier input."""
     rng = np.random.default_rng(21)
@@ -200,6 +260,15 @@ def test_row_programs_match_the_oracle(C, H, T, layers, vocab, gelu, nb, keep):
     b = block(C, H, T, layers, vocab, gelu)
     cm = check(b.module, b.consts, b, block_inputs(b, nb), keep, False)
     assert any(fn is rowprog.call for _, fn, _ in cm.plan(nb, keep).steps)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,H", [(32, 2), (16, 1)])
+@pytest.mark.parametrize("keep", ["outputs", "all"])
+def test_one_row_matches_the_oracle(C, H, keep):
+    b = block(C, H, 1)
+    cm = check(b.module, b.consts, b, block_inputs(b, 1), keep, False)
+    assert any(fn is rowprog.call for _, fn, _ in cm.plan(1, keep).steps)
 
 
 @pytest.mark.gpu
