@@ -318,27 +318,20 @@ def plan(cm, P, prog, views, nb, keep, step) -> bool:
     lay = layout(cm, prog, external)
     if lay is None:
         return False
-    mem = []
-    for d in lay["ops"]:                                    # operands first: nothing is allocated for a program refused
+    mem, results, nbufs = [], {}, len(P.bufs)
+    for d in lay["ops"]:                                    # operands and stored results
+        m = None
         if "load" in d:
             m = _memory(views[d["load"]], rows, d["n"])
-            if m is None:
-                return False
-            mem.append(m)
-        else:
-            mem.append(None)
-    for i, d in enumerate(lay["ops"]):
-        if "load" in d:
-            continue
-        r = d["value"]
-        if not d["store"]:
-            continue
-        view = cm._alloc_result(P, r.owner, (nb, *g.qt(r).dims), r.owner.sym_str or "row")
-        views[r] = view
-        if d.get("trans"):
-            mem[i] = (view, view.strides[-1], view.strides[0])
-        else:
-            mem[i] = _memory(view, rows, d["n"])
+        elif d["store"]:
+            r = d["value"]
+            view = results[r] = cm._alloc_result(P, r.owner, (nb, *g.qt(r).dims), r.owner.sym_str or "row")
+            m = (view, view.strides[-1], view.strides[0]) if d.get("trans") else _memory(view, rows, d["n"])
+        if m is None and ("load" in d or d["store"]):       # no rows of one stride: nothing is kept of the program
+            del P.bufs[nbufs:]
+            return False
+        mem.append(m)
+    views.update(results)
     launch = Launch(cm, prog, lay, rows, T, cm._row_stream(lay))
     launch.mem = mem
     step("+".join(op.sym_str or op.name.split(".")[-1] for op in prog.ops), call, cm.dev, launch)

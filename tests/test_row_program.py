@@ -216,6 +216,26 @@ def test_one_row_of_k_blocked_values(monkeypatch, C, H, keep):
         assert any(v.kb for v in cm.plan(1, keep).views.values())
 
 
+def test_a_result_without_rows_of_one_stride_runs_op_by_op(monkeypatch):
+    """A program whose stored result the kernel cannot address is refused whole, and leaves no buffer behind."""
+    dev, memory, refused = RowFake(), rowprog._memory, []
+    monkeypatch.setattr(rt, "device", lambda index=0: dev)
+    b = block(32, 2, 16)
+    op_by_op = anvil_mi355x.compile(b)
+    op_by_op.row_programs = False
+    names = [buf.name for buf in op_by_op.plan(3).bufs]
+
+    def no_results(view, rows, n):
+        if view.buf.name == "out":
+            return refused.append(view)
+        return memory(view, rows, n)
+    monkeypatch.setattr(rowprog, "_memory", no_results)
+    cm = check(b.module, b.consts, b, block_inputs(b, 3), "outputs", False)
+    assert refused and [c[0] for c in dev.calls].count("row_program") == 1
+    names.remove("h1")                                   # inside the first program
+    assert [buf.name for buf in cm.plan(3).bufs] == names
+
+
 def late_graph(late):
     """h = x w, then r = h + z, where z is an input after h, or a view made after h of an earlier input."""
     rng = np.random.default_rng(21)
