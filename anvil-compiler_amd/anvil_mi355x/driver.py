@@ -984,8 +984,9 @@ class CompiledModel:
                 if self.scale(sym) is None:
                     raise ValueError(f"input {sym!r} has no scale: pass integer inputs with quantized=True")
                 # quantized on the device (clamp(rint(x / scale)) in float64, as quantize_input does on the host);
-                # the kernel also flags NaN and infinite values, which upload_inputs turns into the reference's
-                # ValueError (anvil/driver.py:265-266) before the forward is launched
+                # the kernel also flags NaN and infinite values (and stores 0 for them), which run turns into
+                # the reference's ValueError (anvil/driver.py:265-266): upload_inputs before the forward is launched, or,
+                # for the single small input that it leaves to run's next check, the read-back after it
                 out[sym] = _FloatInput(np.ascontiguousarray(v, dtype=np.float32 if v.dtype == np.float32
                                                             else np.float64))
             if not batch:
@@ -1164,6 +1165,16 @@ class CompiledModel:
                 narrow[s] = base if whole else base[0]
         return out
 
+    def _settle(self):
+        """After a run that failed part way: wait until no kernel reads its host input any more, and take the violation
+        that it left on the device (else the next run would report it). Returns that violation, or None."""
+        if hasattr(self.dev, "fetch"):
+            try:
+                self.dev.fetch([])(check=True)
+            except Exception as e:
+                return e
+        return None
+
     AUTO_EAGER_RUNS = 2                # eager runs a plan times before its graph is captured and timed
 
     def _auto_graph(self, plan) -> bool:
@@ -1220,10 +1231,11 @@ class CompiledModel:
                 self.dev.record(3)
                 ints = self.read(plan, syms, nb, batch, narrow, check=True)
             except BaseException as e:
-                if hasattr(self.dev, "fetch"):
-                    self.dev.fetch([])()              # nothing reads this run's host input any more
-                if floats and isinstance(e, ValueError) and "NaN or infinite" in str(e):
-                    raise ValueError(f"input {self.inputs[0]!r} has NaN or infinite values") from None
+                flagged = self._settle()
+                if floats and isinstance(e, Exception):
+                    for seen in (e, flagged):
+                        if isinstance(seen, ValueError) and "NaN or infinite" in str(seen):
+                            raise ValueError(f"input {self.inputs[0]!r} has NaN or infinite values") from None
                 raise
             total_ms = self.dev.elapsed_ms(2, 3)
             if auto:
