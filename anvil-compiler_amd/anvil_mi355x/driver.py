@@ -798,12 +798,15 @@ class CompiledModel:
                 flags |= rt.GEMM_CAUSAL_SKIP
             elif self._causal_k_ok(op):
                 flags |= rt.GEMM_CAUSAL_K
-        # lead dims: broadcast an operand over lead dims it lacks (stride 0)
+        # lead dims: broadcast an operand over lead dims it lacks (stride 0): a const all of them, a computed (K, N) right
+        # operand those after the batch dim
         lc = list(zip(c.dims[:-2], c.strides[:-2]))
-        l1 = list(zip(rows1.dims[:-2], rows1.strides[:-2]))
-        l2 = list(zip(rows2.dims[:-2], rows2.strides[:-2]))
-        l1 = [(d, 0) for d, _ in lc[:len(lc) - len(l1)]] + l1
-        l2 = [(d, 0) for d, _ in lc[:len(lc) - len(l2)]] + l2
+
+        def spread(v, operand):
+            own = list(zip(v.dims[:-2], v.strides[:-2]))
+            at = 0 if operand in self.is_const else 1
+            return own[:at] + [(d, 0) for d, _ in lc[at:at + len(lc) - len(own)]] + own[at:]
+        l1, l2 = spread(rows1, op.b if swapped else op.a), spread(rows2, op.a if swapped else op.b)
         # fold every lead dim into the row dim when rows1 and C allow it and rows2 does not vary over them
         if all(s == 0 for _, s in l2) and not (flags & (rt.GEMM_CAUSAL_SKIP | rt.GEMM_CAUSAL_K)):
             r1 = rows1.reshape((math.prod(rows1.dims[:-1]), K)) if len(rows1.dims) == len(c.dims) else None

@@ -558,3 +558,21 @@ def test_rmsnorm_after_a_fused_add_joins_its_epilogue(fake, cfg4, keep):
     cm3 = anvil_mi355x.compile(models.config(3)[0])
     cm3._ensure_device()
     assert not any(lab.endswith("+h2") for lab, _, _ in cm3._plan(2, "outputs").steps)
+
+
+@pytest.mark.parametrize("H,nb", [(3, 2), (2, 2), (2, 1), (1, 3)])
+@pytest.mark.parametrize("head_merge", [False, True])
+def test_a_computed_right_operand_is_shared_by_the_heads(fake, H, nb, head_merge):
+    """(H, M, K) @ (K, N), both computed: each sequence's right operand is the same for all of its heads (the stand-in
+    refuses operand ranges that leave their allocation)."""
+    rng = np.random.default_rng([41, H, nb])
+    bld = GraphBuilder("g")
+    o = bld.qmatmul("o", bld.input("a", [H, 8, 32]), bld.input("b", [32, 16]), 3, 13)
+    bld.output(bld.reshape("m", bld.transpose("t", o, [1, 0, 2]), [8, H * 16]) if head_merge else o)
+    m = bld.module()
+    x = {"a": rng.integers(-128, 128, (nb, H, 8, 32)), "b": rng.integers(-128, 128, (nb, 32, 16))}
+    got = anvil_mi355x.compile(m).run([x["a"], x["b"]], "mi355x", batch=True, quantized=True, keep="all")
+    for i in range(nb):
+        want = interp.run(m, {k: v[i] for k, v in x.items()}, {}).values
+        for k in got.ints:
+            assert np.array_equal(got.ints[k][i], want[k]), (i, k)
