@@ -1,8 +1,10 @@
 // Context, memory, timing and error reporting of the anvil_mi355x C ABI.
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <utility>
 #include <vector>
@@ -33,39 +35,96 @@ struct LaunchList {
   bool incomplete = false;             // a launch could not be noted
 };
 
-// the lists this thread is recording, innermost last, each with the stream it records
+// The recordings under way in the order they began. Each notes the launches that the thread which began it makes on its
+// stream. A capture may end on another thread and a context may be destroyed with recordings open, so they are held for
+// all threads; g_recording, their number, keeps launches outside of any recording from taking the lock.
 struct Recording {
   hipStream_t stream;
+  unsigned long long thread;
+  bool capture;
   LaunchList* list;
 };
-static thread_local std::vector<Recording> g_recordings;
+static std::mutex g_recordings_lock;
+static std::vector<Recording> g_recordings;
+static std::atomic<int> g_recording{0};
+
+static unsigned long long this_thread() {            // never given twice, unlike a thread id
+  static std::atomic<unsigned long long> next{1};
+  static thread_local unsigned long long id = next++;
+  return id;
+}
+
+static bool record_start(hipStream_t s, bool capture) {
+  std::lock_guard<std::mutex> hold(g_recordings_lock);
+  LaunchList* l = new (std::nothrow) LaunchList();
+  if (!l) return false;
+  try {
+    g_recordings.push_back({s, this_thread(), capture, l});
+  } catch (const std::bad_alloc&) {
+    delete l;
+    return false;
+  }
+  ++g_recording;
+  return true;
+}
+
+// The innermost recording of this kind on the stream, ended: a capture's whichever thread began it, a list's on its own
+// thread. Null when there is none.
+static LaunchList* record_stop(hipStream_t s, bool capture) {
+  std::lock_guard<std::mutex> hold(g_recordings_lock);
+  for (size_t i = g_recordings.size(); i-- > 0;) {
+    const Recording r = g_recordings[i];
+    if (r.stream != s || r.capture != capture || (!capture && r.thread != this_thread())) continue;
+    g_recordings.erase(g_recordings.begin() + (long)i);
+    --g_recording;
+    return r.list;
+  }
+  return nullptr;
+}
+
+static void record_drop(hipStream_t s) {             // a destroyed stream's
+  std::lock_guard<std::mutex> hold(g_recordings_lock);
+  for (size_t i = g_recordings.size(); i-- > 0;)
+    if (g_recordings[i].stream == s) {
+      delete g_recordings[i].list;
+      g_recordings.erase(g_recordings.begin() + (long)i);
+      --g_recording;
+    }
+}
+
+static void note(LaunchList& list, const void* sym, dim3 grid, dim3 block, unsigned lds, void** args,
+                 const unsigned short* sizes, int n) {
+  LaunchRecord r{sym, nullptr, grid, block, lds, {}, {}, {sizes, sizes + n}};
+  if (hipGetFuncBySymbol(&r.fn, sym) != hipSuccess) {
+    (void)hipGetLastError();
+    list.incomplete = true;
+    return;
+  }
+  size_t total = 0;
+  for (int i = 0; i < n; ++i) total = (total + 15) / 16 * 16 + sizes[i];
+  r.bytes.resize(total + 1);
+  size_t at = 0;
+  for (int i = 0; i < n; ++i) {
+    at = (at + 15) / 16 * 16;
+    std::memcpy(r.bytes.data() + at, args[i], sizes[i]);
+    r.ptrs.push_back(r.bytes.data() + at);
+    at += sizes[i];
+  }
+  list.launches.push_back(std::move(r));             // moving the vectors keeps their storage, and so the pointers
+}
 
 // A launch that cannot be noted has still run: it only spoils the recordings, which then end in an error.
 static void note_launch(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
-                        const unsigned short* sizes, int n) try {
-  for (Recording& rec : g_recordings) {
-    if (rec.stream != s) continue;
-    LaunchRecord r{sym, nullptr, grid, block, lds, {}, {}, {sizes, sizes + n}};
-    if (hipGetFuncBySymbol(&r.fn, sym) != hipSuccess) {
-      (void)hipGetLastError();
+                        const unsigned short* sizes, int n) {
+  std::lock_guard<std::mutex> hold(g_recordings_lock);
+  for (const Recording& rec : g_recordings) {
+    if (rec.stream != s || rec.thread != this_thread()) continue;
+    try {
+      note(*rec.list, sym, grid, block, lds, args, sizes, n);
+    } catch (const std::bad_alloc&) {
       rec.list->incomplete = true;
-      continue;
     }
-    size_t total = 0;
-    for (int i = 0; i < n; ++i) total = (total + 15) / 16 * 16 + sizes[i];
-    r.bytes.resize(total + 1);
-    size_t at = 0;
-    for (int i = 0; i < n; ++i) {
-      at = (at + 15) / 16 * 16;
-      std::memcpy(r.bytes.data() + at, args[i], sizes[i]);
-      r.ptrs.push_back(r.bytes.data() + at);
-      at += sizes[i];
-    }
-    rec.list->launches.push_back(std::move(r));   // moving the vectors keeps their storage, and so the pointers
   }
-} catch (const std::bad_alloc&) {
-  for (Recording& rec : g_recordings)
-    if (rec.stream == s) rec.list->incomplete = true;
 }
 
 int launch_kernel(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
@@ -78,7 +137,7 @@ int launch_kernel(const void* sym, dim3 grid, dim3 block, unsigned lds, hipStrea
   } else {
     e = hipLaunchKernel(sym, grid, block, args, lds, s);
   }
-  if (e == hipSuccess && !g_recordings.empty()) note_launch(sym, grid, block, lds, s, args, sizes, n);
+  if (e == hipSuccess && g_recording.load(std::memory_order_relaxed)) note_launch(sym, grid, block, lds, s, args, sizes, n);
   return e == hipSuccess ? ANVIL_OK : hip_fail(e, "kernel launch");
 }
 
@@ -218,7 +277,10 @@ int anvil_destroy(anvil_ctx* ctx) {
   if (ctx->host_flags) hipHostFree(ctx->host_flags);
   if (ctx->ws) hipFree(ctx->ws);
   for (int* w : ctx->ws_retired) hipFree(w);
-  if (ctx->stream) hipStreamDestroy(ctx->stream);
+  if (ctx->stream) {
+    record_drop(ctx->stream);
+    hipStreamDestroy(ctx->stream);
+  }
   delete ctx;
   return ANVIL_OK;
 }
@@ -320,26 +382,16 @@ int anvil_zero(anvil_ctx* ctx, void* dst, size_t bytes) {
   return zero_fill(ctx->stream, dst, bytes);
 }
 
-// Recordings start and end on one thread; they nest.
-static void record_start(anvil_ctx* ctx) { g_recordings.push_back({ctx->stream, new LaunchList()}); }
-
-static LaunchList* record_stop(anvil_ctx* ctx) {
-  if (g_recordings.empty() || g_recordings.back().stream != ctx->stream) return nullptr;
-  LaunchList* l = g_recordings.back().list;
-  g_recordings.pop_back();
-  return l;
-}
-
 int anvil_graph_begin(anvil_ctx* ctx) {
   if (int r = check_ctx(ctx)) return r;
   ANVIL_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
-  record_start(ctx);
+  (void)record_start(ctx->stream, true);                 // without a list the capture keeps its executable form
   return ANVIL_OK;
 }
 
 int anvil_graph_end(anvil_ctx* ctx, void** graph) {
   if (int r = check_ctx(ctx)) return r;
-  LaunchList* l = record_stop(ctx);
+  LaunchList* l = record_stop(ctx->stream, true);
   if (!graph) {
     delete l;
     return set_error(ANVIL_E_VALUE, "anvil_graph_end: null output pointer");
@@ -351,14 +403,18 @@ int anvil_graph_end(anvil_ctx* ctx, void** graph) {
     delete l;
     return hip_fail(e, "hipStreamEndCapture(ctx->stream, &g)");
   }
-  // The captured nodes are this thread's recorded launches, one after another on one stream: they are replayed as
-  // launches from the list. hipGraphLaunch of the same kernels costs more on both sides: 28 us of host time for one
+  // Where the captured nodes are the noted launches of the thread that began, one after another on one stream, they are
+  // replayed as launches from the list. hipGraphLaunch of the same kernels costs more on both sides: 28 us of host time for one
   // node to 43 us for twelve, and about 0.7 us more a node on the device (measured: a 768-wide block on one sequence,
   // 7 nodes, 61.4 us a forward through hipGraphLaunch, 55 us as launches; the 128-wide two-layer model, 12 nodes,
   // 96.5 against 89.7 us). A graph that holds anything else keeps its executable form.
   size_t nodes = 0;
   e = hipGraphGetNodes(g, nullptr, &nodes);
-  if (!l) l = new LaunchList();
+  if (!l) l = new (std::nothrow) LaunchList();
+  if (!l) {
+    hipGraphDestroy(g);
+    return set_error(ANVIL_E_RUNTIME, "anvil_graph_end: out of memory");
+  }
   if (e != hipSuccess || nodes != l->launches.size() || l->incomplete) {
     l->launches.clear();
     e = hipGraphInstantiate(&l->exec, g, nullptr, nullptr, 0);
@@ -374,13 +430,13 @@ int anvil_graph_end(anvil_ctx* ctx, void** graph) {
 
 int anvil_record_begin(anvil_ctx* ctx) {
   if (int r = check_ctx(ctx)) return r;
-  record_start(ctx);
+  if (!record_start(ctx->stream, false)) return set_error(ANVIL_E_RUNTIME, "anvil_record_begin: out of memory");
   return ANVIL_OK;
 }
 
 int anvil_record_end(anvil_ctx* ctx, void** list) {
   if (int r = check_ctx(ctx)) return r;
-  LaunchList* l = record_stop(ctx);
+  LaunchList* l = record_stop(ctx->stream, false);
   if (!list) {
     delete l;
     return set_error(ANVIL_E_VALUE, "anvil_record_end: null output pointer");
@@ -403,7 +459,7 @@ int anvil_graph_launch(anvil_ctx* ctx, void* graph) {
     ANVIL_HIP(hipGraphLaunch(l->exec, ctx->stream));
     return ANVIL_OK;
   }
-  const bool plain = g_recordings.empty() && !(g_timer.stop && g_timer.stream == ctx->stream);
+  const bool plain = !g_recording.load(std::memory_order_relaxed) && !(g_timer.stop && g_timer.stream == ctx->stream);
   for (LaunchRecord& r : l->launches) {
     if (plain) {
       ANVIL_HIP(hipModuleLaunchKernel(r.fn, r.grid.x, r.grid.y, r.grid.z, r.block.x, r.block.y, r.block.z, r.lds,

@@ -74,16 +74,17 @@ int anvil_zero(anvil_ctx* ctx, void* dst, size_t bytes);
  * recorded with), and anvil_graph_destroy frees. Between begin and end, call only op entry points whose workspace is
  * already allocated (run the same calls once first): anvil_upload, anvil_download, anvil_sync and a first-use
  * allocation end the capture with an error. The library's kernels clear memory with fill kernels, never
- * hipMemsetAsync, so a capture holds kernel nodes only, all of them launched by the calling thread: it is replayed as
- * launches of those kernels from native code, which costs less than hipGraphLaunch of the same nodes on the host and
- * between the kernels. (A capture that holds anything else is replayed as an executable HIP graph.) */
+ * hipMemsetAsync, so a capture holds kernel nodes only. When the thread that began it launched all of them, it is replayed
+ * as launches of those kernels from native code, which costs less than hipGraphLaunch of the same nodes on the host and
+ * between the kernels; any other capture is replayed as an executable HIP graph. Any thread may end a capture. */
 int anvil_graph_begin(anvil_ctx* ctx);
 int anvil_graph_end(anvil_ctx* ctx, void** graph);
 int anvil_graph_launch(anvil_ctx* ctx, void* graph);
 int anvil_graph_destroy(anvil_ctx* ctx, void* graph);
 /* The same list of launches taken while they run: the kernels that this thread's op calls launch on the context's
  * stream between anvil_record_begin and anvil_record_end run as usual and are noted in *list, which
- * anvil_graph_launch and anvil_graph_destroy take. Only kernels are noted, no copy and no synchronisation. */
+ * anvil_graph_launch and anvil_graph_destroy take. Only kernels are noted, no copy and no synchronisation. The thread that
+ * began a recording ends it; anvil_destroy drops a context's open recordings. */
 int anvil_record_begin(anvil_ctx* ctx);
 int anvil_record_end(anvil_ctx* ctx, void** list);
 
