@@ -97,3 +97,37 @@ def test_batched_and_grouped_products(dev):
     assert np.array_equal(out[0].download((B, T, C), np.int8), y[0])
     assert np.array_equal(out[1].download((B, C, T), np.int8), y[1].transpose(0, 2, 1))
     assert np.array_equal(out[2].download((B, T, 70), np.int8), y[2][..., :70])
+
+
+# Past two 64 x 64 tiles a CU (512 on 256 CUs) the one-tile-per-workgroup kernels take the same calls: 128 x 128 tiles
+# with ragged rows and columns, K below, at and past their stages of 64 bytes, whole rotations of three stages (192) or not
+
+@pytest.mark.parametrize("M,N,K", [(2080, 1030, 16), (2049, 1090, 48), (4100, 600, 144), (2177, 1040, 192), (2100, 1100, 1008),
+                                   (8193, 300, 384), (2177, 1152, 256)])
+@pytest.mark.parametrize("form", ["plain", "kblocked", "lut", "i16"])
+@pytest.mark.parametrize("mul24", [True, False])
+def test_products_past_the_line(dev, M, N, K, form, mul24):
+    assert -(-M // 64) * -(-N // 64) > 512
+    test_products(dev, M, N, K, form, mul24)
+
+
+@pytest.mark.parametrize("M,N,K,ldr", [(2080, 1040, 64, 1040), (2049, 1090, 272, 1090), (4100, 592, 192, 608)])
+@pytest.mark.parametrize("store_y", [True, False])
+@pytest.mark.parametrize("ma,mb,s2", [(300, -200, 9), (16777216, -16777216, 25)])
+def test_residual_add_past_the_line(dev, M, N, K, ldr, store_y, ma, mb, s2):
+    test_residual_add(dev, M, N, K, ldr, store_y, ma, mb, s2)
+
+
+@pytest.mark.parametrize("B,H,T,d", [(40, 4, 100, 64), (70, 2, 130, 48)])
+def test_batched_products_past_the_line(dev, B, H, T, d):
+    """scores = q k^T of every head, read in place: batch strides (T C, d), row stride C."""
+    rng = np.random.default_rng([57, B, T])
+    C = H * d
+    q, k = rng.integers(-128, 128, (2, B, T, C))
+    S = dev.alloc(B * H * T * T)
+    dev.gemm_i8(up(dev, q), up(dev, k), S, B, H, T, T, d, [T * C, d, C, T * C, d, C, H * T * T, T * T, T], MULT, SHIFT, None,
+                "i8", rt.GEMM_UNCHECKED | rt.GEMM_MUL24)
+    dev.sync()
+    heads = lambda a: a.reshape(B, T, H, d).transpose(0, 2, 1, 3)                 # noqa: E731
+    want = sem.qmatmul(heads(q), heads(k).swapaxes(-1, -2), MULT, SHIFT, fast=True)
+    assert np.array_equal(S.download((B, H, T, T), np.int8), want)

@@ -1,4 +1,4 @@
-"""Split-K GEMMs (ANVIL_GEMM_SPLITK, and the library's own choice for few-tile products) against the oracle and the
+"""Split-K GEMMs (ANVIL_GEMM_SPLITK) and the few-tile products that used to split by themselves, against the oracle and the
 one-pass kernels: same bits, on ragged shapes, i16 results, LUT epilogues and the 24-bit requant, run repeatedly so
 that a workspace left dirty by one call would show up in the next (reference op: anvil/semantics.py:95-103)."""
 import numpy as np
@@ -60,8 +60,8 @@ def test_forced_split_k_matches_oracle_and_one_pass(dev, M, K, N, dtype, lut):
 
 
 def test_few_tile_products_repeat_exactly(dev):
-    """The config-2 shape 256 x 3072 x 3072 takes split-K by itself (256 x 768 x 768 does not); ten calls in a row
-    give the same bits."""
+    """Few-tile products that the library gives to one kernel (config 2's 256 x 3072 x 3072 and 256 x 768 x 768); ten calls
+    in a row give the same bits."""
     for K in (768, 3072):
         a, w, m, s, table, want, _ = _case(256, K, K, 7)
         for _ in range(10):
