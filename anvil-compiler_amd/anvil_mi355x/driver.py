@@ -116,12 +116,12 @@ class _Plan:
         self.host_in: dict = {}        # page-locked inputs of run(), by sym
         self.reads: dict = {}          # read()'s buffers by its syms
         self.host_stage: dict = {}     # page-locked host buffers the read-back downloads into, by device buffer
-        self.graph = None              # the steps captured as one HIP graph (run(..., graph=True))
+        self.graph = None              # the captured forward (run(..., graph=True))
         self.launched = False          # an eager launch has run
         self.sequence = None           # the kernels of the plan's second eager launch, for the next ones
         self.eager_ms: list = []       # device ms of the plan's first eager runs (run's default launch choice)
         self.graph_ms = None           # device ms of its first replay of the captured graph
-        self.replay = None             # run's choice once measured: True = replay the graph, False = launch eagerly
+        self.replay = None             # run's choice once measured: True = replay the capture, False = launch()
         self.kb_values: set = set()    # values stored K-blocked (read only by GEMMs)
 
     def buf(self, nbytes, name=""):
@@ -1084,11 +1084,11 @@ class CompiledModel:
         return b
 
     def launch(self, plan, profile=False, graph=False):
-        """Enqueue every kernel of the plan on the device stream (asynchronous unless profile). The plan's
-        first two launches call its steps one by one, the second recording the kernels they launch (Device.sequence);
-        the next ones issue those kernels in one native call. graph=True replays the steps as captured on the plan's first such launch, right
-        after an ordinary launch of the same steps (which allocates every workspace they need, so the capture records
-        kernels only)."""
+        """Enqueue every kernel of the plan on the device stream (asynchronous unless profile). The plan's first two
+        launches call its steps one by one, the second recording the kernels they launch (Device.sequence); the next
+        ones issue those kernels in one native call. graph=True replays the steps as captured on the plan's first such
+        launch, right after an ordinary launch of the same steps (which allocates every workspace they need, so the
+        capture records kernels only)."""
         times = {}
         if not profile and graph:
             if plan.graph is None:
@@ -1138,12 +1138,13 @@ class CompiledModel:
         return fetch, pinned, plain
 
     def read(self, plan, syms, nb=None, batch=True, narrow=None, check=False) -> dict:
-        """sym -> int64 array of each of syms, read back from the device; check: as the device's sync() reports
-        violations, first. Device buffers of up to PINNED_MAX bytes are copied into page-locked buffers of the plan, with
-        one wait for all of them (Device.fetch), and widened from there, while the plan's page-locked buffers stay within PINNED_PLAN_MAX bytes in total; beyond that a
-        read downloads into ordinary (pageable) memory. With a dict `narrow`, also sym -> the same values as a view at their stored dtype (no copy, into
-        that buffer: use it before the plan's next read). Reads of one plan from several threads need the device
-        lock around them, as run() holds it."""
+        """sym -> int64 array of each of syms, read back from the device; check: violations are reported first, as the
+        device's sync() reports them (a non-finite float input before any other). Device buffers of up to PINNED_MAX
+        bytes are copied into page-locked buffers of the plan, with one wait for all of them (Device.fetch), and widened
+        from there, while the plan's page-locked buffers stay within PINNED_PLAN_MAX bytes in total; beyond that a read
+        downloads into ordinary (pageable) memory. With a dict `narrow`, also sym -> the same values as a view at their
+        stored dtype (no copy, into that buffer: use it before the plan's next read). Reads of one plan from several
+        threads need the device lock around them, as run() holds it."""
         got = plan.reads.get(tuple(syms))
         if got is None:
             got = plan.reads[tuple(syms)] = self._read_buffers(plan, syms)
@@ -1178,12 +1179,13 @@ class CompiledModel:
                 return e
         return None
 
-    AUTO_EAGER_RUNS = 2                # eager runs a plan times before its graph is captured and timed
+    AUTO_EAGER_RUNS = 2                # runs a plan times before its forward is captured and the replay timed
 
     def _auto_graph(self, plan) -> bool:
-        """run's default launch: a plan's first AUTO_EAGER_RUNS runs launch eagerly, the next captures the steps
-        as a HIP graph (after running them once more), the one after replays it; from then on the faster of the
-        two, compared on the device time of the forward (launch gaps included)."""
+        """run's default launch: a plan's first AUTO_EAGER_RUNS runs call its steps one by one, the next captures them
+        (after running them once more), the one after replays the capture. From then on the replay, if it took less
+        device time (launch gaps included) than the first runs, else launch(), which by then issues the same kernels
+        from its own recorded list: the two cost alike, and only steps that cannot be replayed faster keep launch()."""
         if plan.replay is not None:
             return plan.replay
         return len(plan.eager_ms) >= self.AUTO_EAGER_RUNS
@@ -1203,10 +1205,11 @@ class CompiledModel:
             tokens=False, graph=None, **run_kw) -> RunOutput:
         """Quantize x (unless quantized=True), run the graph on the GPU, read back (reference driver.py:305-322).
         Float inputs are quantized on the device. tokens=True: x holds token ids of a model compiled with embedding
-        tables, gathered and quantized on the device. graph=True runs the forward as one HIP graph of the plan
-        (captured on first use): the same kernels with no launch gaps between them; graph=False launches every kernel
-        from the host; graph=None (the default) measures both on the plan's first runs and keeps the faster
-        (small batches gain most: their kernels are short and the launch gaps between them a large share)."""
+        tables, gathered and quantized on the device. graph=True replays the plan's captured forward (captured on first
+        use): the same kernels issued in one native call; graph=False launches them through launch(), which calls the
+        steps one by one twice and issues its recorded list from then on; graph=None (the default) times the first runs
+        and a replay and goes on with the faster (_auto_graph). result["hip_graph"] says that this run replayed the
+        capture, which runs as an executable HIP graph only when it holds more than this thread's launches."""
         if backend not in BACKENDS:
             raise ValueError(f"unknown backend {backend!r}: {', '.join(BACKENDS)}")
         if run_kw:

@@ -11,7 +11,6 @@ from dataclasses import dataclass
 
 import numpy as np
 
-
 ITEMSIZE = {"i8": 1, "i16": 2, "i32": 4}
 
 

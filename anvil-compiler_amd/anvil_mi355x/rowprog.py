@@ -50,11 +50,12 @@ class Program:
 
 def _product_min(rows) -> int:
     """The bound on the smaller of a product's K and N. A program trades launches for a chain of ops that each wave runs
-    in turn, so it gains where its products are small: 32-wide blocks (hidden width 128) took 19 us against 21 op by op
-    at 16 rows, 27 against 46 at 65,536 and 116 against 207 in two layers of 131,072; the frozen 32-wide models 39
-    against 57 at 32 rows and 123 against 242 at 262,144. 64-wide blocks gain once four row blocks a CU (on 256) hide
-    the chain: 46 against 56 at 32,768 rows (42 against 46 in longer sequences), but 30 against 25 at 32 rows and 31
-    against 26 at 2,048. From widths of 96 on programs lost at every size."""
+    in turn, so it gains where its products are small. Measured on 256 CUs: 32-wide blocks (hidden width 128) took 19 us
+    against 21 op by op at 16 rows, 27 against 46 at 65,536 and 116 against 207 in two layers of 131,072; the frozen
+    32-wide models 39 against 57 at 32 rows and 123 against 242 at 262,144. 64-wide blocks gain once four row blocks a CU
+    hide the chain: 46 against 56 at 32,768 rows (42 against 46 in longer sequences), but 30 against 25 at 32 rows and 31
+    against 26 at 2,048; between those two the line was not measured. From widths of 96 on programs lost at every
+    size."""
     return 64 if rows >= 32768 else 32
 
 

@@ -295,9 +295,9 @@ class Device:
         return HostBuffer(self, nbytes)
 
     def capture(self, fn, *args) -> HipGraph:
-        """fn(*args) recorded as a HIP graph of this context's stream instead of run (anvil_graph_begin / _end): the
-        op calls it makes must need no first-use allocation and no synchronisation. The capture ends whatever fn
-        raises."""
+        """fn(*args) captured on this context's stream instead of run (anvil_graph_begin / _end), for launch() of the
+        result to replay: the op calls it makes must need no first-use allocation and no synchronisation. The capture
+        ends whatever fn raises."""
         self.lib.call("anvil_graph_begin", self.ctx)
         handle = C.c_void_p()
         try:

@@ -70,7 +70,7 @@ struct KernelTimer {
 extern __thread KernelTimer g_timer;   // zero-initialised per thread (a trivial type: no TLS init function)
 
 // Every kernel goes out through launch_kernel: with the timer's events while it is armed for the stream, and noted in
-// the launch list that this thread is recording on the stream, if any (anvil_graph_begin, anvil_record_begin).
+// the launch lists that this thread has begun to record on the stream, if any (anvil_graph_begin, anvil_record_begin).
 int launch_kernel(const void* fn, dim3 grid, dim3 block, unsigned lds, hipStream_t s, void** args,
                   const unsigned short* sizes, int n);
 

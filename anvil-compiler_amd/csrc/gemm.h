@@ -1,5 +1,5 @@
-// What the GEMM kernels (gemm.hip, gemm_deep.hip, gemm_any.hip) share: their arguments, LDS swizzle, direct-to-LDS loads, waits, and the
-// register epilogue.
+// What the GEMM kernels (gemm.hip, gemm_deep.hip, gemm_any.hip) share: their arguments, LDS swizzle, direct-to-LDS
+// loads, waits, and the register epilogue.
 #pragma once
 
 #include <type_traits>

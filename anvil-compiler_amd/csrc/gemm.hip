@@ -1438,8 +1438,8 @@ struct Prepared {
 // the time. Measured (128 x 128 tiles or the kernels that served few tiles before -> 64 x 64 deep): 1024 x 768 x 768 with
 // its add 7.5 -> 5.0 us, 1024 x 768 x 3072 with its add 15.6 -> 9.3, 256 x 3072 x 3072 9.9 -> 8.7, 2048 x 1024 x 768 (two
 // tiles a CU) 6.9 -> 6.0; past two tiles a CU it loses: three 1024 x 768 x 768 (576 tiles) 7.7 -> 9.3, 4608 x 512 x 512
-// with its add (576) 7.5 -> 8.1. The same line holds where two stages take all of K: 16384 x 512 x 128 (2048 tiles) 5.9 ->
-// 8.6, 65536 x 128 x 128 (2048) 5.9 -> 8.5, 16384 x 256 x 256 (1024) 5.3 -> 5.8; only N that half
+// with its add (576) 7.5 -> 8.1. The same line holds for the two-stage form (K up to 256): 16384 x 512 x 128 (2048 tiles)
+// 5.9 -> 8.6, 65536 x 128 x 128 (2048) 5.9 -> 8.5, 16384 x 256 x 256 (1024) 5.3 -> 5.8; only N that half
 // fills its last 128 columns gains past it (16384 x 192 x 192, 768 tiles, 6.3 -> 4.8; its whole block stayed within noise).
 static bool deep_ok(const Prepared& p) {
   return p.fast && p.g.causal == 0 && !(p.g.res && p.osz == 2) && (!p.g.res || 64 * p.g.ldr < (1ll << 31));
@@ -1447,8 +1447,8 @@ static bool deep_ok(const Prepared& p) {
 static long long deep_tiles(const Prepared& p) {
   return (long long)((p.g.M + 63) / 64) * ((p.g.N + 63) / 64) * p.batch;
 }
-// two stages hold all of K up to 256 (and leave LDS for four workgroups a CU): 2048 x 1024 x 128 with its add 4.7 against
-// 5.0 us on four stages; from 512 on four are faster (5.9 against 6.2 us)
+// K up to 256 is two stages, which leave LDS for four workgroups a CU but have one stage in flight: 2048 x 1024 x 128
+// with its add 4.7 against 5.0 us on four stages; from K = 512 on four are faster (5.9 against 6.2 us)
 static int deep_stages(int K) { return K <= 256 ? 2 : 4; }
 
 // Argument checks that need no context (a group checks every member before any launch).

@@ -3,9 +3,12 @@
 // What bounds them: not MFMAs and not bandwidth but the latency of the operand loads. After a kernel boundary the XCD's L2
 // holds none of the operands, a load takes about a microsecond, and a K loop that keeps two stages of 64 K bytes in flight
 // pays that latency once every two stages: 1024 x 768 x 3072 on 128 x 128 tiles took 15.6 us with its residual add,
-// 1024 x 768 x 768 7.5 us. These kernels keep three stages of 128 K bytes in flight (NS = 4, two workgroups a CU), or for
-// K up to 256 all of K (NS = 2), on 64 x 64 tiles, which spread the same product over four times the CUs: 9.3 and 5.0 us.
-// (Eight stages, one workgroup a CU: 9.5 and 5.6 us; 128 x 128 tiles with four stages: 16.4 and 8.8 us.)
+// 1024 x 768 x 768 7.5 us. These kernels keep three stages of 128 K bytes in flight (NS = 4, two workgroups a CU), on 64 x
+// 64 tiles, which spread the same product over four times the CUs: 9.3 and 5.0 us. (Eight stages, one workgroup a CU: 9.5
+// and 5.6 us, so past three stages load latency is no longer all of it: with one workgroup a CU a stage is also a chain of
+// fragment reads, four MFMAs on one accumulator, a wait and a barrier. 128 x 128 tiles with four stages: 16.4 and 8.8 us.)
+// K up to 256 takes NS = 2: one stage in flight, issued before the stage in LDS is used, so that K's two stages arrive one
+// after the other; what hides their latency is the four workgroups a CU that its LDS leaves room for.
 //
 // One workgroup of four waves (2 x 2) per BM x BN tile, direct-to-LDS loads as in fast_tile (gemm.hip), stage s in array
 // s % NS. The waves walk the stages with one barrier a stage. Bt rows enter LDS in bperm order, so a lane's accumulators

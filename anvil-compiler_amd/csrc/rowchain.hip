@@ -4,7 +4,7 @@
 //
 // What bounds them: at small widths each op alone is a launch of 4 us or more whose time is its latency (dispatch, the
 // first loads, a K loop of one or two steps, the stores) and a pass of the activations through memory; a row needs none
-// of the other rows, so a wave can take its rows through all of the ops. A program is bound by its epilogues instead: on
+// of the other rows, so a wave can take its rows through all of the ops. What is left is mostly its epilogues: on
 // the 32-wide frozen model's 262,144 rows of int16 the middle program (y .. mlp .. next q, k, v: 19 ops) takes 45 us, of
 // which 50 MB in and out are 10 and its MFMA 2; whole model 242 -> 123 us, at 32 rows 57 -> 39.
 //

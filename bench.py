@@ -14,8 +14,8 @@ kernel trace. --config 1, 3, 4 run the other blocks; --config 2 the standalone i
 Printed: one JSON line with the metric, the dominant kernel's roofline, a per-kernel breakdown from an untimed
 profiled pass (kernel-bound events again, so the figures add up to less than ms_per_step), a stream-copy figure for
 the achievable HBM bandwidth, the PCIe-inclusive rate of `cm.run` on the host float input (never `value`), the step
-time of the same kernels replayed as one captured HIP graph (`hip_graph`; `value` takes the faster of the eager and
-the replayed step, as cm.run does by default, and `launch` names it), and the
+time of the same kernels replayed from one capture (`hip_graph`: launches issued by one native call a forward; `value`
+takes the faster of the eager and the replayed step, and `launch` names it), and the
 CPU baseline: this repo's literal numpy restatement of the reference interpreter (oracle/, int64 `@`, single-threaded
 per process) on P sequences of the same batch in P processes on this host's cores (exact, as batched evaluation
 equals per-sample evaluation), scaled to tokens/s. It runs before the GPU is first touched, so the worker processes
@@ -176,7 +176,7 @@ def bench_block(args):
     wall_s, device_ms, dom_us, n, dom2_us, n2 = timed_steps(dev, steps, K, dom, dom2)
     per = kernel_times(dev, steps)           # after the timed steps: the clock has settled
     graph = graph_steps(cm, plan, K)
-    # cm.run's default launch (driver.CompiledModel._auto_graph): the faster of eager launches and the captured graph
+    # op by op from Python, or the captured forward by one native call a step
     eager_ms = wall_s / K * 1e3
     mode = "graph" if graph["ms_per_step"] < eager_ms else "eager"
     step_ms = min(eager_ms, graph["ms_per_step"])
@@ -243,8 +243,7 @@ def bench_block(args):
                    "graph_ms_per_step": graph["ms_per_step"], "steps": K,
                    "covers": "value and ms_per_step: the faster of the two timed regions, each K steps between device "
                              "synchronisations (host wall clock): eager launches (where the roofline kernels carry "
-                             "their events) and the same kernels replayed as one captured HIP graph; cm.run keeps the "
-                             "faster of the two by default"},
+                             "their events) and the captured forward's kernels replayed by one native call a step"},
         "end_to_end": e2e,
         "hip_graph": graph,
         "kernels": kernels,
@@ -542,9 +541,9 @@ def cpu_baseline(built, xq, outs):
 
 
 def graph_steps(cm, plan, K):
-    """The same forward replayed as one HIP graph of the plan (cm.launch(plan, graph=True), captured on first use):
-    K replays between device synchronisations, host wall clock. `value` takes it when it is faster than the eager
-    launches, as cm.run does by default."""
+    """The same forward replayed from the plan's capture (cm.launch(plan, graph=True), captured on first use): K
+    replays between device synchronisations, host wall clock. `value` takes it when it is faster than the eager
+    launches."""
     cm.launch(plan, graph=True)
     cm.dev.sync()
     t0 = time.perf_counter()
@@ -553,7 +552,7 @@ def graph_steps(cm, plan, K):
     cm.dev.sync()
     dt = time.perf_counter() - t0
     return {"ms_per_step": round(dt / K * 1e3, 4), "steps": K,
-            "covers": "the timed forward's kernels replayed as one captured HIP graph (run(..., graph=True))"}
+            "covers": "the timed forward's kernels replayed from its capture (run(..., graph=True))"}
 
 
 def end_to_end(cm, x, nb, seq, keep, calls=3):
